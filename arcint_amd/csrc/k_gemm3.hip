@@ -1,6 +1,7 @@
 // k_gemm3.hip - the streaming prefill GEMMs on gfx950 v_mfma_i32_32x32x32_i8: Q4_K
 // (k_gemm3_q4k, also the grouped MoE GEMM) and the block types with one float scale per 32
-// weights, Q4_0, Q8_0 and IQ4_NL (k_gemm3_blk), weights streamed by each wave.
+// weights, Q4_0, Q8_0 and IQ4_NL (k_gemm3_blk), weights streamed by each wave; one product, or a
+// gate/up pair with its GLU in one launch (PAIR).
 //
 // Role of the reference's int8 prefill GEMMs (kernel_mul_mm_kq2d_q4_0_i8, P0099:377-455;
 // kernel_mul_mm_kq2d_q4_K_i8, P01:1919-2024) and its fp16 tile kernel for Q8_0
@@ -37,6 +38,7 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 namespace qmm {
 namespace {
@@ -127,12 +129,13 @@ struct KQParams {
     const float * dcol;                  // [column][nsb]
     const int8_t * bsp;                  // [super-block][ldT][16]
     int64_t ldk, ldT, ncols;
-    // grouped mode with a GLU (glu >= 0): this launch is the up product, gsrc the gate product's
-    // rows at the same offsets; stores act(gate) * up.  dspan: floats of dst (and gsrc) the
-    // stores may reach, below 2^30
-    const float * gsrc;
-    int glu;
+    // grouped mode: floats of dst the stores may reach, below 2^30
     int64_t dspan;
+    // a gate/up pair (up != nullptr): w is the gate's image, up the up matrix's (same shape and
+    // type); even waves of a slice take the gate's row halves, odd ones the same row halves of
+    // up, and the odd ones store act(gate) * up, act = glu (QMM_GLU_*)
+    const uint8_t * up;
+    int glu;
 };
 
 // The work-group's block L and K piece (-1: the whole K) from its index bx.  Blocks [0, full)
@@ -152,37 +155,44 @@ __device__ __forceinline__ bool kq_block(const KQParams & p, uint32_t bx, uint32
     return e < (uint32_t)(p.total - p.full) * (uint32_t)p.ts;
 }
 
-// The ts pieces of a tail block add a wave's 32 sums per lane (out0, out1) up a pairwise tree of
+// The ts pieces of a tail block add a column tile's 16 sums per lane up a pairwise tree of
 // exchanges in slot memory, as the split GEMV's K slices do: at a level of n nodes, node i meets
 // node i ^ 1 in slot i / 2 of the level (an odd last node moves up alone); the first arrival
 // leaves its value and drops it, the second adds it to its own (a + b = b + a: the same sum
 // whichever arrives first) and puts the slot back to kTreeEmpty.  Returns the mask of values
 // this lane still holds at the root (to be stored); every slot ends empty.  nodes: the wave's
-// slots, [slot][32 values][64 lanes].
-__device__ __forceinline__ uint32_t kq_meet(uint32_t * nodes, int piece, int ts, v16f & out0, v16f & out1,
-                                            int lane) {
-    uint32_t live = 0xffffffffu;
+// slots, [slot][32 values][64 lanes], at this tile's first value.  A gate/up pair's two sums (PAIR:
+// g the gate's) travel as one 64-bit value.
+template <bool PAIR>
+__device__ __forceinline__ uint32_t kq_meet(uint32_t * nodes, int piece, int ts, float (&g)[16], float (&v)[16], int lane) {
+    typedef std::conditional_t<PAIR, unsigned long long, uint32_t> word;
+    constexpr word kEmpty = PAIR ? (word)(((unsigned long long)kTreeEmpty << 32) | kTreeEmpty) : (word)kTreeEmpty;
+    uint32_t live = 0xffffu;
     uint32_t i = (uint32_t)piece, n = (uint32_t)ts, off = 0;
     while (n > 1) {                                               // uniform
         if ((i ^ 1u) < n) {
-            uint32_t * sl = nodes + (size_t)(off + (i >> 1)) * 2048 + lane;
-            uint32_t o[32];
+            word * sl = reinterpret_cast<word *>(nodes) + (size_t)(off + (i >> 1)) * 2048 + lane;
+            word o[16];
 #pragma unroll
-            for (int r = 0; r < 32; ++r) {
-                const float v = r < 16 ? out0[r] : out1[r - 16];
-                o[r] = (live >> r) & 1u ? __hip_atomic_exchange(sl + r * 64, __float_as_uint(v), __ATOMIC_RELAXED,
-                                                                __HIP_MEMORY_SCOPE_AGENT)
-                                        : kTreeEmpty;
+            for (int r = 0; r < 16; ++r) {
+                word x = __float_as_uint(v[r]);
+                if constexpr (PAIR) x = (x << 32) | __float_as_uint(g[r]);
+                o[r] = (live >> r) & 1u ? __hip_atomic_exchange(sl + r * 64, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                        : kEmpty;
             }
 #pragma unroll
-            for (int r = 0; r < 32; ++r) {
+            for (int r = 0; r < 16; ++r) {
                 if (!((live >> r) & 1u)) continue;
-                if (o[r] == kTreeEmpty) {
+                if (o[r] == kEmpty) {
                     live &= ~(1u << r);
                 } else {
-                    if (r < 16) out0[r] += __uint_as_float(o[r]);
-                    else out1[r - 16] += __uint_as_float(o[r]);
-                    __hip_atomic_store(sl + r * 64, kTreeEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if constexpr (PAIR) {
+                        g[r] += __uint_as_float((uint32_t)o[r]);
+                        v[r] += __uint_as_float((uint32_t)(o[r] >> 32));
+                    } else {
+                        v[r] += __uint_as_float(o[r]);
+                    }
+                    __hip_atomic_store(sl + r * 64, kEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
             }
         }
@@ -195,9 +205,19 @@ __device__ __forceinline__ uint32_t kq_meet(uint32_t * nodes, int piece, int ts,
 
 // v[i] = act(g[i]) * v[i] for one GLU op, as the split GLU computes it (glu_apply)
 template <int OP>
-__device__ __forceinline__ void glu_rows(const float (&g)[32], float (&v)[32]) {
+__device__ __forceinline__ void glu_rows(const float (&g)[16], float (&v)[16]) {
 #pragma unroll
-    for (int i = 0; i < 32; ++i) v[i] = glu_apply(OP, g[i], v[i]);
+    for (int i = 0; i < 16; ++i) v[i] = glu_apply(OP, g[i], v[i]);
+}
+// one branch for the op, then straight-line code over the values
+__device__ __forceinline__ void glu_switch(int op, const float (&g)[16], float (&v)[16]) {
+    switch (op) {
+        case QMM_GLU_REGLU: glu_rows<QMM_GLU_REGLU>(g, v); break;
+        case QMM_GLU_GEGLU: glu_rows<QMM_GLU_GEGLU>(g, v); break;
+        case QMM_GLU_SWIGLU: glu_rows<QMM_GLU_SWIGLU>(g, v); break;
+        case QMM_GLU_GEGLU_ERF: glu_rows<QMM_GLU_GEGLU_ERF>(g, v); break;
+        default: glu_rows<QMM_GLU_GEGLU_QUICK>(g, v); break;
+    }
 }
 
 // the two 16-bit halves of v times those of s (v_pk_mul_lo_u16)
@@ -225,46 +245,135 @@ __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, uint8_t * lds, u
                                              0, 0);
 }
 
-// Grouped mode's store of a wave's 32 sums per lane (rows m, the unit's 64 slots): each output
-// goes to its pair's dst offset, read from the unit.  Every offset (and gate value) is requested
-// before the first store, and no load or store sits in a branch: through buffer resources over
-// dst's span an offset past it (kNoStore: a slot past the unit) reads zero and drops its store.
-// (Conditional accesses, and loads after stores to dst that might alias them, made each of the 32
-// stores wait for a memory round trip.)  With p.glu >= 0 the launch is the up product of a
-// gate/up pair: act(gate) * up, gate read at the same offset.
-__device__ __forceinline__ void gather_store(const KQParams & p, uint32_t nb, int ncu, int64_t m, int h,
-                                             const v16f & out0, const v16f & out1) {
-    constexpr uint32_t kNoStore = 0xffffffffu;
-    const uint32_t span4 = (uint32_t)(p.dspan * 4);
-    const __amdgpu_buffer_rsrc_t dres = buffer_rsrc(p.dst, span4);
-    uint32_t off[32];
-    float val[32];
-#pragma unroll
-    for (int i = 0; i < 32; ++i) {
-        const int slot = 32 * (i >> 4) + 8 * ((i & 15) >> 2) + 4 * h + (i & 3);   // < 64: in the unit
-        const int64_t o = p.units[nb].c[slot].dst_off + m;
-        off[i] = slot < ncu ? 4u * (uint32_t)o : kNoStore;
-        val[i] = i < 16 ? out0[i] : out1[i - 16];
-    }
-    if (p.glu >= 0) {                                         // uniform
-        const __amdgpu_buffer_rsrc_t gres = buffer_rsrc(p.gsrc, span4);
-        float gv[32];
-#pragma unroll
-        for (int i = 0; i < 32; ++i) gv[i] = __uint_as_float(bld4(gres, off[i], 0));
-        // one branch for the op, then straight-line code over the values
-        switch (p.glu) {
-            case QMM_GLU_REGLU: glu_rows<QMM_GLU_REGLU>(gv, val); break;
-            case QMM_GLU_GEGLU: glu_rows<QMM_GLU_GEGLU>(gv, val); break;
-            case QMM_GLU_SWIGLU: glu_rows<QMM_GLU_SWIGLU>(gv, val); break;
-            case QMM_GLU_GEGLU_ERF: glu_rows<QMM_GLU_GEGLU_ERF>(gv, val); break;
-            default: glu_rows<QMM_GLU_GEGLU_QUICK>(gv, val); break;
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 32; ++i) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(val[i]), dres, (int)off[i], 0, 0);
+// Where a wave stands: its work-group's block (mb, nb), its row half, and which matrix of a gate/up
+// pair it takes.  Row-half waves u of a slice: U row halves, or U / 2 of both matrices (even waves
+// the gate's, odd ones up's, the same row half, so that the two sums meet inside the work-group).
+struct KQWave {
+    int64_t rh, mtile;
+    const uint8_t * base;
+    int t;
+    bool row_ok;                                              // a missing row half computes a copy, stores nothing
+};
+template <bool PAIR>
+__device__ __forceinline__ KQWave kq_wave(const KQParams & p, uint32_t mb, int U, int u) {
+    KQWave v;
+    const int64_t raw = PAIR ? (int64_t)mb * (U / 2) + (u >> 1) : (int64_t)mb * U + u;
+    v.row_ok = raw < 2 * p.w.ntiles;
+    v.rh = v.row_ok ? raw : 2 * p.w.ntiles - 1;
+    v.mtile = v.rh >> 1;
+    v.t = (int)(v.rh & 1);
+    v.base = PAIR && (u & 1) ? p.up : p.w.base;
+    return v;
 }
 
-template <int U, bool GATHER>
+// The end of a block, a wave's 32 sums per lane (row m, the column pair's two tiles) complete over
+// its K slice:
+//  * K slices 1.. add theirs into slice 0's through LDS, in slice order;
+//  * a gate/up pair: the gate's waves hand their sums to up's through LDS (no product of the pair
+//    is written to memory and read back, and no GLU launch follows).  Against two launches and a GLU
+//    kernel (grouped: the gate's rows through memory): Q4_0 2 x 11008 x 4096 at 2048 columns 237 x 2 +
+//    62 -> 492 us, Q4_K 2 x 17408 x 5120 at 512 111 x 2 + 26 -> 234, at 77 42 x 2 + 6 -> 75; 128 experts
+//    512 x 2048 of 64 pairs each 64 x 2 -> 80 us.  A template argument: as a run-time branch its code
+//    cost the single products 0.8 us a launch (4 % of a 20 us one) in instruction fetch;
+//  * a tail piece's sums meet its partners' in tree slots, the holder of a sum stores it;
+//  * the store: dense, each value to its column (non-temporal); grouped, to its pair's dst offset,
+//    read from the unit: every offset is requested before the first store, and through a buffer
+//    resource over dst's span an offset past it (kNoStore: a slot past the unit) drops its store,
+//    so no store sits in a branch or waits for a load.
+// Every wave of the work-group calls it (it holds barriers).
+template <bool GATHER, bool PAIR>
+__device__ __forceinline__ void kq_finish(const KQParams & p, uint8_t * lds, uint32_t L, int piece, uint32_t nb, uint32_t i2,
+                                          uint32_t i3, int U, int u, int ks, bool row_ok, int64_t m, int ncu, float scale,
+                                          v16f & out0, v16f & out1) {
+    const int lane = threadIdx.x & 63, h = lane >> 5;
+    float * red = reinterpret_cast<float *>(lds);
+    if (p.KS > 1) {
+        if (ks > 0) {
+            float * o = red + ((size_t)((ks - 1) * U + u) * 32) * 64 + lane;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                o[r * 64] = out0[r];
+                o[(16 + r) * 64] = out1[r];
+            }
+        }
+        __syncthreads();
+        if (ks == 0) {
+            for (int k = 1; k < p.KS; ++k) {
+                const float * o = red + ((size_t)((k - 1) * U + u) * 32) * 64 + lane;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    out0[r] += o[r * 64];
+                    out1[r] += o[(16 + r) * 64];
+                }
+            }
+        }
+        if constexpr (PAIR) __syncthreads();                  // (the slices' sums are read: the pair's go there)
+    }
+    [[maybe_unused]] const float * x = red + (size_t)(u >> 1) * 2048 + lane;
+    if constexpr (PAIR) {
+        if (ks == 0 && !(u & 1)) {
+            float * o = red + (size_t)(u >> 1) * 2048 + lane;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                o[r * 64] = out0[r];
+                o[(16 + r) * 64] = out1[r];
+            }
+        }
+        __syncthreads();
+        if (!(u & 1)) return;
+    }
+    if (ks > 0 || !row_ok || m >= p.w.M) return;
+    // (one column tile at a time: at 168 registers the pairs of both tiles would spill)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        float gv[16], val[16];
+        uint32_t live = 0xffffu;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) val[r] = c ? out1[r] : out0[r];
+        if constexpr (PAIR) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) gv[r] = x[(16 * c + r) * 64];
+            if (piece >= 0)
+                live = kq_meet<true>(p.tree + (((size_t)(L - p.full) * (U / 2) + (u >> 1)) * (size_t)p.tslots * 2048 +
+                                               (size_t)c * 1024) * 2, piece, p.ts, gv, val, lane);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                gv[r] *= scale;
+                val[r] *= scale;
+            }
+            glu_switch(p.glu, gv, val);
+        } else {
+            if (piece >= 0)
+                live = kq_meet<false>(p.tree + ((size_t)(L - p.full) * U + u) * (size_t)p.tslots * 2048 + (size_t)c * 1024, piece,
+                                      p.ts, gv, val, lane);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) val[r] *= scale;
+        }
+        if constexpr (GATHER) {
+            constexpr uint32_t kNoStore = 0xffffffffu;
+            const __amdgpu_buffer_rsrc_t dres = buffer_rsrc(p.dst, (uint32_t)(p.dspan * 4));
+            uint32_t off[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int slot = 32 * c + 8 * (r >> 2) + 4 * h + (r & 3);   // < 64: in the unit
+                const int64_t o = p.units[nb].c[slot].dst_off + m;
+                off[r] = slot < ncu ? 4u * (uint32_t)o : kNoStore;
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(val[r]), dres, (int)off[r], 0, 0);
+        } else {
+            float * dst = p.dst + (int64_t)i2 * p.bt.d_nb2 + (int64_t)i3 * p.bt.d_nb3 + m;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int64_t n = (2 * (int64_t)nb + c) * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+                if (n < p.N && ((live >> r) & 1u)) __builtin_nontemporal_store(val[r], dst + n * p.bt.d_nb1);
+            }
+        }
+    }
+}
+
+template <int U, bool GATHER, bool PAIR>
 __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_q4k(KQParams p) {
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, j32 = lane & 31;
@@ -284,11 +393,12 @@ __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_q4k(KQParams p) {
         mat = __builtin_amdgcn_readfirstlane(p.units[nb].mat);
         ncu = __builtin_amdgcn_readfirstlane(p.units[nb].ncols);
     }
-    const int64_t rh_raw = (int64_t)mb * U + u;               // the wave's row half
-    const bool row_ok = rh_raw < 2 * p.w.ntiles;              // a missing row half computes a copy, stores nothing
-    const int64_t rh = row_ok ? rh_raw : 2 * p.w.ntiles - 1;
-    const int64_t mtile = rh >> 1;
-    const int t = (int)(rh & 1);
+    const KQWave wv = kq_wave<PAIR>(p, mb, U, u);
+    const bool row_ok = wv.row_ok;
+    const int64_t mtile = wv.mtile;
+    const int t = wv.t;
+    WView ww = p.w;
+    ww.base = wv.base;
     const int64_t ct0 = (int64_t)bz * p.ntb + 2 * (int64_t)nb; // the pair's first column tile
     const int64_t nct = std::min<int64_t>(2, p.ntb - 2 * (int64_t)nb);
     const int nsb = (int)p.nsb;
@@ -300,12 +410,12 @@ __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_q4k(KQParams p) {
 
     if (GATHER && mat < 0) {                                  // invalid ids: zero rows (uniform)
         const int64_t m = mtile * kTileRows + 32 * t + j32;
-        if (!row_ok || m >= p.w.M || ks > 0) return;
+        if (!row_ok || m >= p.w.M || ks > 0 || (PAIR && !(u & 1))) return;
         for (int n = h; n < ncu; n += 2) p.dst[p.units[nb].c[n].dst_off + m] = 0.0f;
         return;
     }
 
-    const __amdgpu_buffer_rsrc_t wbuf = buffer_rsrc(tile_group(p.w, mat, mtile, 0), (uint32_t)(p.w.G * p.w.tg));
+    const __amdgpu_buffer_rsrc_t wbuf = buffer_rsrc(tile_group(ww, mat, mtile, 0), (uint32_t)(p.w.G * p.w.tg));
     // the pair's activations; a pair with one tile reads zeros for the second (past the range);
     // grouped mode: the whole quantization, each lane at its own column (zeros past the unit)
     const __amdgpu_buffer_rsrc_t abuf = GATHER ? buffer_rsrc(p.codes, (uint32_t)(p.ncols * p.ldk))
@@ -518,50 +628,8 @@ __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_q4k(KQParams p) {
         __syncthreads();
     }
 
-    // ---- K slices 1.. add their sums into slice 0's through LDS (fixed order), slice 0 stores
-    if (p.KS > 1) {
-        float * red = reinterpret_cast<float *>(lds);
-        if (ks > 0) {
-            float * o = red + ((size_t)((ks - 1) * U + u) * 32) * 64 + lane;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                o[r * 64] = out0[r];
-                o[(16 + r) * 64] = out1[r];
-            }
-        }
-        __syncthreads();
-        if (ks > 0) return;
-        for (int k = 1; k < p.KS; ++k) {
-            const float * o = red + ((size_t)((k - 1) * U + u) * 32) * 64 + lane;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                out0[r] += o[r * 64];
-                out1[r] += o[(16 + r) * 64];
-            }
-        }
-    }
-    if (!row_ok) return;
-    const int64_t m = mtile * kTileRows + 32 * t + j32;
-    if (m >= p.w.M) return;
-    if constexpr (GATHER) {
-        gather_store(p, nb, ncu, m, h, out0, out1);
-        return;
-    }
-    // a tail piece: the block's pieces meet first, the holder of a sum stores it
-    const uint32_t live = piece >= 0 ? kq_meet(p.tree + ((size_t)(L - p.full) * U + u) * (size_t)p.tslots * 2048, piece,
-                                               p.ts, out0, out1, lane)
-                                     : 0xffffffffu;
-    float * dst = p.dst + (int64_t)i2 * p.bt.d_nb2 + (int64_t)i3 * p.bt.d_nb3 + m;
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        const int64_t n0 = (2 * (int64_t)nb + c) * 32;
-        const v16f & v = c ? out1 : out0;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int64_t n = n0 + 8 * (r >> 2) + 4 * h + (r & 3);
-            if (n < p.N && ((live >> (16 * c + r)) & 1u)) __builtin_nontemporal_store(v[r], dst + n * p.bt.d_nb1);
-        }
-    }
+    kq_finish<GATHER, PAIR>(p, lds, L, piece, nb, i2, i3, U, u, ks, row_ok, mtile * kTileRows + 32 * t + j32, ncu,
+              1.0f, out0, out1);
 }
 
 // ---- Q6_K ------------------------------------------------------------------------------------
@@ -584,7 +652,7 @@ __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_q4k(KQParams p) {
 //    nibble for s < 2, high for s >= 2) with qh[32 n + l] bits 2 s, 2 s + 1 above it; lane half
 //    h holds l in [16 h, 16 h + 16): ql chunk plane 4 n + 2 (s & 1) + h, qh plane 8 + 2 n + h.
 //  * Per super-block and output: out += dx (d isum) (ggml's d_w d_x times the integer sum).
-template <int U, bool GATHER>
+template <int U, bool GATHER, bool PAIR>
 __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_q6k(KQParams p) {
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, j32 = lane & 31;
@@ -604,11 +672,12 @@ __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_q6k(KQParams p) {
         mat = __builtin_amdgcn_readfirstlane(p.units[nb].mat);
         ncu = __builtin_amdgcn_readfirstlane(p.units[nb].ncols);
     }
-    const int64_t rh_raw = (int64_t)mb * U + u;               // the wave's row half
-    const bool row_ok = rh_raw < 2 * p.w.ntiles;              // a missing row half computes a copy, stores nothing
-    const int64_t rh = row_ok ? rh_raw : 2 * p.w.ntiles - 1;
-    const int64_t mtile = rh >> 1;
-    const int t = (int)(rh & 1);
+    const KQWave wv = kq_wave<PAIR>(p, mb, U, u);
+    const bool row_ok = wv.row_ok;
+    const int64_t mtile = wv.mtile;
+    const int t = wv.t;
+    WView ww = p.w;
+    ww.base = wv.base;
     const int64_t ct0 = (int64_t)bz * p.ntb + 2 * (int64_t)nb; // the pair's first column tile
     const int64_t nct = std::min<int64_t>(2, p.ntb - 2 * (int64_t)nb);
     const int nsb = (int)p.nsb;
@@ -619,12 +688,12 @@ __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_q6k(KQParams p) {
 
     if (GATHER && mat < 0) {                                  // invalid ids: zero rows (uniform)
         const int64_t m = mtile * kTileRows + 32 * t + j32;
-        if (!row_ok || m >= p.w.M || ks > 0) return;
+        if (!row_ok || m >= p.w.M || ks > 0 || (PAIR && !(u & 1))) return;
         for (int n = h; n < ncu; n += 2) p.dst[p.units[nb].c[n].dst_off + m] = 0.0f;
         return;
     }
 
-    const __amdgpu_buffer_rsrc_t wbuf = buffer_rsrc(tile_group(p.w, mat, mtile, 0), (uint32_t)(p.w.G * p.w.tg));
+    const __amdgpu_buffer_rsrc_t wbuf = buffer_rsrc(tile_group(ww, mat, mtile, 0), (uint32_t)(p.w.G * p.w.tg));
     // (grouped mode: the route's whole quantization, each lane at its own column, as k_gemm3_q4k)
     const __amdgpu_buffer_rsrc_t abuf = GATHER ? buffer_rsrc(p.codes, (uint32_t)(p.ncols * p.ldk))
                                                : buffer_rsrc(p.tA + ct0 * p.nsb * 8192, (uint32_t)(nct * p.nsb * 8192));
@@ -808,49 +877,8 @@ __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_q6k(KQParams p) {
         __syncthreads();
     }
 
-    // ---- K slices 1.. add their sums into slice 0's through LDS (fixed order), slice 0 stores
-    if (p.KS > 1) {
-        float * red = reinterpret_cast<float *>(lds);
-        if (ks > 0) {
-            float * o = red + ((size_t)((ks - 1) * U + u) * 32) * 64 + lane;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                o[r * 64] = out0[r];
-                o[(16 + r) * 64] = out1[r];
-            }
-        }
-        __syncthreads();
-        if (ks > 0) return;
-        for (int k = 1; k < p.KS; ++k) {
-            const float * o = red + ((size_t)((k - 1) * U + u) * 32) * 64 + lane;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                out0[r] += o[r * 64];
-                out1[r] += o[(16 + r) * 64];
-            }
-        }
-    }
-    if (!row_ok) return;
-    const int64_t m = mtile * kTileRows + 32 * t + j32;
-    if (m >= p.w.M) return;
-    if constexpr (GATHER) {
-        gather_store(p, nb, ncu, m, h, out0, out1);
-        return;
-    }
-    const uint32_t live = piece >= 0 ? kq_meet(p.tree + ((size_t)(L - p.full) * U + u) * (size_t)p.tslots * 2048, piece,
-                                               p.ts, out0, out1, lane)
-                                     : 0xffffffffu;
-    float * dst = p.dst + (int64_t)i2 * p.bt.d_nb2 + (int64_t)i3 * p.bt.d_nb3 + m;
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        const int64_t n0 = (2 * (int64_t)nb + c) * 32;
-        const v16f & v = c ? out1 : out0;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int64_t n = n0 + 8 * (r >> 2) + 4 * h + (r & 3);
-            if (n < p.N && ((live >> (16 * c + r)) & 1u)) __builtin_nontemporal_store(v[r], dst + n * p.bt.d_nb1);
-        }
-    }
+    kq_finish<GATHER, PAIR>(p, lds, L, piece, nb, i2, i3, U, u, ks, row_ok, mtile * kTileRows + 32 * t + j32, ncu,
+              1.0f, out0, out1);
 }
 
 // ---- IQ4_XS and Q5_K: one integer scale per 32-weight sub-block ----------------------------
@@ -870,7 +898,7 @@ __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_q6k(KQParams p) {
 //    planes 9 + h (bit j of byte l: the fifth bit of weight l of sub-block j); codes 0..31; the
 //    min term as k_gemm3_q4k's (two MFMAs per column tile over the split sums and the mins).
 //  * Per super-block and output: out += dx (d isum) (IQ4_XS), dx (d isum - dmin imn) (Q5_K).
-template <int TYPE, int U, bool GATHER>
+template <int TYPE, int U, bool GATHER, bool PAIR>
 __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_sbs(KQParams p) {
     constexpr bool Q5 = TYPE == QMM_TYPE_Q5_K;
     constexpr int kVm = Q5 ? (6 | (0x7 << 4) | (0xF << 8)) : (10 | (0x7 << 4) | (0xF << 8));   // weight loads a super-block
@@ -892,11 +920,12 @@ __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_sbs(KQParams p) {
         mat = __builtin_amdgcn_readfirstlane(p.units[nb].mat);
         ncu = __builtin_amdgcn_readfirstlane(p.units[nb].ncols);
     }
-    const int64_t rh_raw = (int64_t)mb * U + u;               // the wave's row half
-    const bool row_ok = rh_raw < 2 * p.w.ntiles;              // a missing row half computes a copy, stores nothing
-    const int64_t rh = row_ok ? rh_raw : 2 * p.w.ntiles - 1;
-    const int64_t mtile = rh >> 1;
-    const int t = (int)(rh & 1);
+    const KQWave wv = kq_wave<PAIR>(p, mb, U, u);
+    const bool row_ok = wv.row_ok;
+    const int64_t mtile = wv.mtile;
+    const int t = wv.t;
+    WView ww = p.w;
+    ww.base = wv.base;
     const int64_t ct0 = (int64_t)bz * p.ntb + 2 * (int64_t)nb; // the pair's first column tile
     const int64_t nct = std::min<int64_t>(2, p.ntb - 2 * (int64_t)nb);
     const int nsb = (int)p.nsb;
@@ -907,12 +936,12 @@ __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_sbs(KQParams p) {
 
     if (GATHER && mat < 0) {                                  // invalid ids: zero rows (uniform)
         const int64_t m = mtile * kTileRows + 32 * t + j32;
-        if (!row_ok || m >= p.w.M || ks > 0) return;
+        if (!row_ok || m >= p.w.M || ks > 0 || (PAIR && !(u & 1))) return;
         for (int n = h; n < ncu; n += 2) p.dst[p.units[nb].c[n].dst_off + m] = 0.0f;
         return;
     }
 
-    const __amdgpu_buffer_rsrc_t wbuf = buffer_rsrc(tile_group(p.w, mat, mtile, 0), (uint32_t)(p.w.G * p.w.tg));
+    const __amdgpu_buffer_rsrc_t wbuf = buffer_rsrc(tile_group(ww, mat, mtile, 0), (uint32_t)(p.w.G * p.w.tg));
     // (grouped mode: the route's whole quantization, each lane at its own column, as k_gemm3_q4k)
     const __amdgpu_buffer_rsrc_t abuf = GATHER ? buffer_rsrc(p.codes, (uint32_t)(p.ncols * p.ldk))
                                                : buffer_rsrc(p.tA + ct0 * p.nsb * 8192, (uint32_t)(nct * p.nsb * 8192));
@@ -1143,49 +1172,8 @@ __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_sbs(KQParams p) {
         __syncthreads();
     }
 
-    // ---- K slices 1.. add their sums into slice 0's through LDS (fixed order), slice 0 stores
-    if (p.KS > 1) {
-        float * red = reinterpret_cast<float *>(lds);
-        if (ks > 0) {
-            float * o = red + ((size_t)((ks - 1) * U + u) * 32) * 64 + lane;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                o[r * 64] = out0[r];
-                o[(16 + r) * 64] = out1[r];
-            }
-        }
-        __syncthreads();
-        if (ks > 0) return;
-        for (int k = 1; k < p.KS; ++k) {
-            const float * o = red + ((size_t)((k - 1) * U + u) * 32) * 64 + lane;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                out0[r] += o[r * 64];
-                out1[r] += o[(16 + r) * 64];
-            }
-        }
-    }
-    if (!row_ok) return;
-    const int64_t m = mtile * kTileRows + 32 * t + j32;
-    if (m >= p.w.M) return;
-    if constexpr (GATHER) {
-        gather_store(p, nb, ncu, m, h, out0, out1);
-        return;
-    }
-    const uint32_t live = piece >= 0 ? kq_meet(p.tree + ((size_t)(L - p.full) * U + u) * (size_t)p.tslots * 2048, piece,
-                                               p.ts, out0, out1, lane)
-                                     : 0xffffffffu;
-    float * dst = p.dst + (int64_t)i2 * p.bt.d_nb2 + (int64_t)i3 * p.bt.d_nb3 + m;
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        const int64_t n0 = (2 * (int64_t)nb + c) * 32;
-        const v16f & v = c ? out1 : out0;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int64_t n = n0 + 8 * (r >> 2) + 4 * h + (r & 3);
-            if (n < p.N && ((live >> (16 * c + r)) & 1u)) __builtin_nontemporal_store(v[r], dst + n * p.bt.d_nb1);
-        }
-    }
+    kq_finish<GATHER, PAIR>(p, lds, L, piece, nb, i2, i3, U, u, ks, row_ok, mtile * kTileRows + 32 * t + j32, ncu,
+              1.0f, out0, out1);
 }
 
 // ---- Q4_0, Q8_0, IQ4_NL: the streaming form with 32-row x 64-column waves -----------------
@@ -1207,7 +1195,7 @@ __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_sbs(KQParams p) {
 //    accumulates it (ggml's per-block combine);
 //  * the lane's weights stream one group ahead: a block's chunk is reloaded with the next
 //    group's as soon as its MFMAs are issued.
-template <int TYPE, int U>
+template <int TYPE, int U, bool PAIR>
 __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_blk(KQParams p) {
     constexpr bool Q8 = TYPE == QMM_TYPE_Q8_0;
     constexpr bool NLQ = TYPE == QMM_TYPE_IQ4_NL;
@@ -1224,11 +1212,12 @@ __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_blk(KQParams p) {
     const uint32_t bz = blockIdx.y;
     const uint32_t i2 = bz % (uint32_t)p.bt.ne12, i3 = bz / (uint32_t)p.bt.ne12;
     const int64_t mat = (int64_t)(i2 / (uint32_t)p.bt.r2) + (int64_t)(i3 / (uint32_t)p.bt.r3) * p.bt.ne02;
-    const int64_t rh_raw = (int64_t)mb * U + u;               // the wave's row half
-    const bool row_ok = rh_raw < 2 * p.w.ntiles;              // a missing row half computes a copy, stores nothing
-    const int64_t rh = row_ok ? rh_raw : 2 * p.w.ntiles - 1;
-    const int64_t mtile = rh >> 1;
-    const int t = (int)(rh & 1);
+    const KQWave wv = kq_wave<PAIR>(p, mb, U, u);
+    const bool row_ok = wv.row_ok;
+    const int64_t mtile = wv.mtile;
+    const int t = wv.t;
+    WView ww = p.w;
+    ww.base = wv.base;
     const int64_t ct0 = (int64_t)bz * p.ntb + 2 * (int64_t)nb; // the pair's first column tile
     const int64_t nct = std::min<int64_t>(2, p.ntb - 2 * (int64_t)nb);
     const int ng = (int)p.nsb;                                // groups (256 weights) along K
@@ -1239,7 +1228,7 @@ __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_blk(KQParams p) {
     const int s1 = std::min(s0 + sps, ke);                    // (every slice has groups)
     const int64_t nblk = 8 * p.nsb;                           // blocks per activation column
 
-    const __amdgpu_buffer_rsrc_t wbuf = buffer_rsrc(tile_group(p.w, mat, mtile, 0), (uint32_t)(p.w.G * p.w.tg));
+    const __amdgpu_buffer_rsrc_t wbuf = buffer_rsrc(tile_group(ww, mat, mtile, 0), (uint32_t)(p.w.G * p.w.tg));
     // the pair's activations; a pair with one tile reads zeros for the second (past the range)
     const __amdgpu_buffer_rsrc_t abuf = buffer_rsrc(p.tA + ct0 * nblk * 1024, (uint32_t)(nct * nblk * 1024));
     const __amdgpu_buffer_rsrc_t dbuf = buffer_rsrc(p.tD + ct0 * nblk * 32, (uint32_t)(nct * nblk * 128));
@@ -1366,143 +1355,51 @@ __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_blk(KQParams p) {
         __syncthreads();
     }
 
-    // ---- K slices 1.. add their sums into slice 0's through LDS (fixed order), slice 0 stores
-    if (p.KS > 1) {
-        float * red = reinterpret_cast<float *>(lds);
-        if (ks > 0) {
-            float * o = red + ((size_t)((ks - 1) * U + u) * 32) * 64 + lane;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                o[r * 64] = out0[r];
-                o[(16 + r) * 64] = out1[r];
-            }
-        }
-        __syncthreads();
-        if (ks > 0) return;
-        for (int k = 1; k < p.KS; ++k) {
-            const float * o = red + ((size_t)((k - 1) * U + u) * 32) * 64 + lane;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                out0[r] += o[r * 64];
-                out1[r] += o[(16 + r) * 64];
-            }
-        }
-    }
-    if (!row_ok) return;
-    const int64_t m = mtile * kTileRows + 32 * t + j32;
-    if (m >= p.w.M) return;
-    const float scale = (TYPE == QMM_TYPE_Q4_0) ? 0.0625f : 1.0f;   // Q4_0 codes carried 16 (q - 8)
-    // a tail piece: the block's pieces meet first, the holder of a sum stores it
-    const uint32_t live = piece >= 0 ? kq_meet(p.tree + ((size_t)(L - p.full) * U + u) * (size_t)p.tslots * 2048, piece,
-                                               p.ts, out0, out1, lane)
-                                     : 0xffffffffu;
-    float * dst = p.dst + (int64_t)i2 * p.bt.d_nb2 + (int64_t)i3 * p.bt.d_nb3 + m;
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        const int64_t n0 = (2 * (int64_t)nb + c) * 32;
-        const v16f & v = c ? out1 : out0;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int64_t n = n0 + 8 * (r >> 2) + 4 * h + (r & 3);
-            if (n < p.N && ((live >> (16 * c + r)) & 1u)) __builtin_nontemporal_store(v[r] * scale, dst + n * p.bt.d_nb1);
-        }
-    }
+    // (Q4_0 codes carried 16 (q - 8))
+    kq_finish<false, PAIR>(p, lds, L, piece, nb, i2, i3, U, u, ks, row_ok, mtile * kTileRows + 32 * t + j32, 0,
+              TYPE == QMM_TYPE_Q4_0 ? 0.0625f : 1.0f, out0, out1);
 }
 
-template <int U, bool GATHER>
-hipError_t launch_kq(const KQParams & q, const G3Shape & sh, const dim3 & g, const dim3 & b, hipStream_t s,
-                     const KTime * kt) {
-    static const hipError_t attr = hipFuncSetAttribute((const void *)k_gemm3_q4k<U, GATHER>,
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    if (attr != hipSuccess) return attr;
-    if (kt) hipExtLaunchKernelGGL(k_gemm3_q4k<U, GATHER>, g, b, (uint32_t)sh.lds, s, kt->start, kt->stop, 0, q);
-    else k_gemm3_q4k<U, GATHER><<<g, b, sh.lds, s>>>(q);
+// one launch of kernel K
+template <typename F>
+hipError_t launch_k(F * k, const KQParams & q, const G3Shape & sh, const dim3 & g, const dim3 & b, hipStream_t s,
+                    const KTime * kt) {
+    if (kt) hipExtLaunchKernelGGL(k, g, b, (uint32_t)sh.lds, s, kt->start, kt->stop, 0, q);
+    else k<<<g, b, sh.lds, s>>>(q);
     return hipGetLastError();
 }
-
-template <int U, bool GATHER>
-hipError_t launch_q6k(const KQParams & q, const G3Shape & sh, const dim3 & g, const dim3 & b, hipStream_t s,
+// (one copy a kernel: its LDS limit is raised once)
+template <int TYPE, int U, bool GATHER, bool PAIR>
+hipError_t launch_one(const KQParams & q, const G3Shape & sh, const dim3 & g, const dim3 & b, hipStream_t s,
                       const KTime * kt) {
-    static const hipError_t attr = hipFuncSetAttribute((const void *)k_gemm3_q6k<U, GATHER>,
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    auto * k = [] {
+        if constexpr (TYPE == QMM_TYPE_Q4_K) return &k_gemm3_q4k<U, GATHER, PAIR>;
+        else if constexpr (TYPE == QMM_TYPE_Q6_K) return &k_gemm3_q6k<U, GATHER, PAIR>;
+        else if constexpr (TYPE == QMM_TYPE_Q5_K || TYPE == QMM_TYPE_IQ4_XS) return &k_gemm3_sbs<TYPE, U, GATHER, PAIR>;
+        else return &k_gemm3_blk<TYPE, U, PAIR>;
+    }();
+    static const hipError_t attr = hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (attr != hipSuccess) return attr;
-    if (kt) hipExtLaunchKernelGGL(k_gemm3_q6k<U, GATHER>, g, b, (uint32_t)sh.lds, s, kt->start, kt->stop, 0, q);
-    else k_gemm3_q6k<U, GATHER><<<g, b, sh.lds, s>>>(q);
-    return hipGetLastError();
+    return launch_k(k, q, sh, g, b, s, kt);
 }
-
-template <int TYPE, int U, bool GATHER>
-hipError_t launch_sbs(const KQParams & q, const G3Shape & sh, const dim3 & g, const dim3 & b, hipStream_t s,
-                      const KTime * kt) {
-    static const hipError_t attr = hipFuncSetAttribute((const void *)k_gemm3_sbs<TYPE, U, GATHER>,
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    if (attr != hipSuccess) return attr;
-    if (kt) hipExtLaunchKernelGGL(k_gemm3_sbs<TYPE, U, GATHER>, g, b, (uint32_t)sh.lds, s, kt->start, kt->stop, 0, q);
-    else k_gemm3_sbs<TYPE, U, GATHER><<<g, b, sh.lds, s>>>(q);
-    return hipGetLastError();
+template <int TYPE, bool GATHER, bool PAIR>
+hipError_t launch_u(const KQParams & q, const G3Shape & sh, const dim3 & g, const dim3 & b, hipStream_t s,
+                    const KTime * kt) {
+    switch (sh.U) {
+        case 12: return launch_one<TYPE, 12, GATHER, PAIR>(q, sh, g, b, s, kt);
+        case 6: return launch_one<TYPE, 6, GATHER, PAIR>(q, sh, g, b, s, kt);
+        case 4: return launch_one<TYPE, 4, GATHER, PAIR>(q, sh, g, b, s, kt);
+        case 3:
+            if constexpr (!PAIR) return launch_one<TYPE, 3, GATHER, PAIR>(q, sh, g, b, s, kt);
+            return hipErrorInvalidValue;                      // (gate and up waves in turn)
+        case 2: return launch_one<TYPE, 2, GATHER, PAIR>(q, sh, g, b, s, kt);
+        default: return hipErrorInvalidValue;
+    }
 }
-
 template <int TYPE, bool GATHER>
-hipError_t launch_sbs_u(const KQParams & q, const G3Shape & sh, const dim3 & g, const dim3 & b, hipStream_t s,
-                        const KTime * kt) {
-    switch (sh.U) {
-        case 12: return launch_sbs<TYPE, 12, GATHER>(q, sh, g, b, s, kt);
-        case 6: return launch_sbs<TYPE, 6, GATHER>(q, sh, g, b, s, kt);
-        case 4: return launch_sbs<TYPE, 4, GATHER>(q, sh, g, b, s, kt);
-        case 3: return launch_sbs<TYPE, 3, GATHER>(q, sh, g, b, s, kt);
-        case 2: return launch_sbs<TYPE, 2, GATHER>(q, sh, g, b, s, kt);
-        default: return hipErrorInvalidValue;
-    }
-}
-
-template <bool GATHER>
-hipError_t launch_q6k_u(const KQParams & q, const G3Shape & sh, const dim3 & g, const dim3 & b, hipStream_t s,
-                        const KTime * kt) {
-    switch (sh.U) {
-        case 12: return launch_q6k<12, GATHER>(q, sh, g, b, s, kt);
-        case 6: return launch_q6k<6, GATHER>(q, sh, g, b, s, kt);
-        case 4: return launch_q6k<4, GATHER>(q, sh, g, b, s, kt);
-        case 3: return launch_q6k<3, GATHER>(q, sh, g, b, s, kt);
-        case 2: return launch_q6k<2, GATHER>(q, sh, g, b, s, kt);
-        default: return hipErrorInvalidValue;
-    }
-}
-
-template <int TYPE, int U>
-hipError_t launch_blk(const KQParams & q, const G3Shape & sh, const dim3 & g, const dim3 & b, hipStream_t s,
-                      const KTime * kt) {
-    static const hipError_t attr = hipFuncSetAttribute((const void *)k_gemm3_blk<TYPE, U>,
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    if (attr != hipSuccess) return attr;
-    if (kt) hipExtLaunchKernelGGL(k_gemm3_blk<TYPE, U>, g, b, (uint32_t)sh.lds, s, kt->start, kt->stop, 0, q);
-    else k_gemm3_blk<TYPE, U><<<g, b, sh.lds, s>>>(q);
-    return hipGetLastError();
-}
-
-template <int TYPE>
-hipError_t launch_blk_u(const KQParams & q, const G3Shape & sh, const dim3 & g, const dim3 & b, hipStream_t s,
-                        const KTime * kt) {
-    switch (sh.U) {
-        case 12: return launch_blk<TYPE, 12>(q, sh, g, b, s, kt);
-        case 6: return launch_blk<TYPE, 6>(q, sh, g, b, s, kt);
-        case 4: return launch_blk<TYPE, 4>(q, sh, g, b, s, kt);
-        case 3: return launch_blk<TYPE, 3>(q, sh, g, b, s, kt);
-        case 2: return launch_blk<TYPE, 2>(q, sh, g, b, s, kt);
-        default: return hipErrorInvalidValue;
-    }
-}
-
-template <bool GATHER>
-hipError_t launch_kq_u(const KQParams & q, const G3Shape & sh, const dim3 & g, const dim3 & b, hipStream_t s,
-                       const KTime * kt) {
-    switch (sh.U) {
-        case 12: return launch_kq<12, GATHER>(q, sh, g, b, s, kt);
-        case 6: return launch_kq<6, GATHER>(q, sh, g, b, s, kt);
-        case 4: return launch_kq<4, GATHER>(q, sh, g, b, s, kt);
-        case 3: return launch_kq<3, GATHER>(q, sh, g, b, s, kt);
-        case 2: return launch_kq<2, GATHER>(q, sh, g, b, s, kt);
-        default: return hipErrorInvalidValue;
-    }
+hipError_t launch_t(const KQParams & q, const G3Shape & sh, const dim3 & g, const dim3 & b, hipStream_t s,
+                    const KTime * kt) {
+    return q.up ? launch_u<TYPE, GATHER, true>(q, sh, g, b, s, kt) : launch_u<TYPE, GATHER, false>(q, sh, g, b, s, kt);
 }
 
 int env_int3(const char * name, int dflt) {
@@ -1531,7 +1428,7 @@ namespace {
 // form, kKQOneSlice); only = -2: every candidate but that one (the grouped mode's split form:
 // there it tied with (2, 2, 3) on 128 experts x 32 pairs and measured 54.8 against 46.8 us)
 constexpr int kKQOneSlice = 4;                                // (4, 1, 3) in the candidates below
-bool kq_shape_ncp(const WView & w, int64_t ncp, int64_t nbatch, G3Shape * sh, bool blk, bool tail, int only) {
+bool kq_shape_ncp(const WView & w, int64_t ncp, int64_t nbatch, G3Shape * sh, bool blk, bool tail, int only, bool pair) {
     struct Cand { int U, KS, per_cu; };
     static const Cand cands[] = { { 12, 1, 1 }, { 6, 2, 1 }, { 4, 3, 1 }, { 3, 4, 1 }, { 4, 1, 3 }, { 2, 2, 3 } };
     const int64_t nrh = 2 * w.ntiles, G = w.G;
@@ -1546,8 +1443,10 @@ bool kq_shape_ncp(const WView & w, int64_t ncp, int64_t nbatch, G3Shape * sh, bo
         // (the block types: two waves per stage share too little of their 2 KB of activations per
         // block; 11008 x 4096 x 512 measured 97 us at (2, 2) against 76 at (12, 1) and (4, 1, 3))
         if (blk && c.U == 2 && forced < 0) continue;
+        if (pair && c.U % 2) continue;                        // (gate and up waves in turn)
         const int64_t sps = (G + c.KS - 1) / c.KS, KS = (G + sps - 1) / sps;
-        const int64_t mbn = (nrh + c.U - 1) / c.U, nwg = mbn * ncp * nbatch;
+        const int rows = pair ? c.U / 2 : c.U;                // row halves of a block
+        const int64_t mbn = (nrh + rows - 1) / rows, nwg = mbn * ncp * nbatch;
         const int64_t slots = (int64_t)cus * c.per_cu;
         // (in 1/64 rounds)
         const int64_t rounds = c.per_cu > 1 ? std::max<int64_t>(64, (nwg * 64 + slots - 1) / slots)
@@ -1571,6 +1470,7 @@ bool kq_shape_ncp(const WView & w, int64_t ncp, int64_t nbatch, G3Shape * sh, bo
     sh->nst = (int)G;
     sh->threads = 64 * sh->U * sh->KS;
     sh->lds = std::max(sh->KS * 2 * kKQStage + (18 % sh->U ? 1024 : 0), (sh->KS - 1) * sh->U * 32 * 64 * 4);
+    if (pair) sh->lds = std::max(sh->lds, sh->U / 2 * 32 * 64 * 4);   // (the gate's sums)
     // The blocks past a whole number per CU (one K slice, one batch) run as ts pieces along K.
     // The hardware puts a block where one finishes, so each CU runs nwg / CUs whole blocks and
     // the remainder would keep nwg % CUs CUs a whole block longer than the rest.  ts minimizes
@@ -1611,7 +1511,83 @@ bool kq_shape_ncp(const WView & w, int64_t ncp, int64_t nbatch, G3Shape * sh, bo
     return sh->mbn * ncp < 0x7fffffff && sh->lds <= 160 * 1024 && sh->threads <= 64 * kKQMaxWaves;
 }
 bool kq_shape(const WView & w, int64_t N, int64_t nbatch, G3Shape * sh, bool blk) {
-    return kq_shape_ncp(w, ((N + 31) / 32 + 1) / 2, nbatch, sh, blk, true, -1);
+    return kq_shape_ncp(w, ((N + 31) / 32 + 1) / 2, nbatch, sh, blk, true, -1, false);
+}
+
+// Launch shape of a dense gate/up pair and its estimated time in us (kernel only), the smallest of
+// the candidates': steps along K of the busiest CU times a step's time.
+//  * A step (256 weights of a wave's 32 rows x 64 columns) takes c us when three waves share a SIMD
+//    3.26 ways, and less than a third as much alone: one wave waits for its next step's weights
+//    (t: 2.0, 2.4, 3.26 c for 1, 2, 3 waves a SIMD; c = 1.1 us for the super-block types, 1.3 for
+//    the 32-weight ones).
+//  * 12-wave blocks run one a CU in whole rounds, 4-wave ones up to three a CU.
+//  * One-slice launches of a block per CU or more may run the blocks past a whole number per CU as
+//    2-4 pieces along K: the pieces' sums pass through memory as 64-bit exchanges, 1.6 us a MB (11008 x
+//    4096 Q4_0, N = 203: 704 pieces, 98 us, against 68 us with 12-wave whole blocks).
+// Measured at (U, KS) = (12, 1) / (6, 2) / (4, 3) / (4, 1) / (2, 2), op us, the estimate's choice first
+// or within 4 % of it: Q4_K 17408 x 5120, N = 77 186 / 90 / 100 / 75 / 83, N = 203 152 / 139 / 166 /
+// 130 / 144, N = 512 247 / 274 / 305 / 234 / 276; Q4_0 11008 x 4096, N = 40 66 / 39 / 31 / 59 / 33, N =
+// 77 64 / 40 / 56 / 45 / 52; IQ4_XS 14336 x 4096, N = 40 74 / 46 / 36 / 45 / 38.
+bool kq_pair_shape(const WView & w, int64_t N, int64_t nbatch, G3Shape * sh, bool blk, double * us) {
+    struct Cand { int U, KS, per_cu; };
+    static const Cand cands[] = { { 12, 1, 1 }, { 6, 2, 1 }, { 4, 3, 1 }, { 4, 1, 3 }, { 2, 2, 3 } };
+    const int64_t ncp = ((N + 31) / 32 + 1) / 2, nrh = 2 * w.ntiles, G = w.G, cus = 256;
+    const int forced = env_int3("QMM_GEMM3_PAIR", -1);         // index into cands (tuning)
+    const double c = blk ? 1.3 : 1.1;
+    auto t = [](double waves) { return waves <= 1 ? 2.0 : waves <= 2 ? 1.6 + 0.4 * waves : 0.68 + 0.86 * waves; };
+    double best = -1;
+    for (int i = 0; i < (int)(sizeof(cands) / sizeof(cands[0])); ++i) {
+        if (forced >= 0 && i != forced) continue;
+        const Cand & cd = cands[i];
+        const int64_t sps = (G + cd.KS - 1) / cd.KS, KS = (G + sps - 1) / sps;
+        const int64_t mbn = (nrh + cd.U / 2 - 1) / (cd.U / 2), nwg = mbn * ncp * nbatch, full = nwg / cus, rest = nwg % cus;
+        auto steps = [&](double load) {                        // of the busiest CU, load blocks on it
+            if (cd.per_cu == 1) return load * ((double)sps * t(cd.U * (double)KS / 4) + 2.0);
+            const double at = std::min(load, (double)cd.per_cu);
+            return (double)sps * t(at * cd.U * (double)KS / 4) * (load / at);
+        };
+        // (two waves share a stage: little beside the waits of up to two blocks a CU)
+        const double two = cd.U == 2 ? (full + (rest > 0) > 2 ? 1.25 : 1.1) : 1.0;
+        double cost = steps((double)(full + (rest > 0))) * c * two;
+        int64_t ts = 1;
+        if (KS == 1 && nbatch == 1 && full > 0) {
+            for (int64_t k = 2; k <= 4 && rest > 0; ++k) {
+                const int64_t pk = (G + k - 1) / k;
+                if (pk < 2 || (k - 1) * pk >= G) continue;
+                const double load = (double)full + (double)((rest * k + cus - 1) / cus) / (double)k;
+                const double v = steps(load) * c + (double)(rest * k) * (cd.U / 2) * 0.026;
+                if (v < cost) {
+                    cost = v;
+                    ts = k;
+                }
+            }
+        }
+        if (best >= 0 && cost >= best) continue;
+        best = cost;
+        *sh = G3Shape{};
+        sh->C = 2;
+        sh->R = 32;
+        sh->SB = 8;
+        sh->U = cd.U;
+        sh->KS = (int)KS;
+        sh->sps = (int)sps;
+        sh->nst = (int)G;
+        sh->mbn = mbn;
+        sh->nbn = ncp;
+        sh->threads = 64 * cd.U * (int)KS;
+        // the stages, or the slices' sums, or the gate's
+        sh->lds = std::max({ (int)KS * 2 * kKQStage + (18 % cd.U ? 1024 : 0), ((int)KS - 1) * cd.U * 32 * 64 * 4,
+                             cd.U / 2 * 32 * 64 * 4 });
+        sh->ts = (int)ts;
+        sh->pk = (int)((G + ts - 1) / ts);
+        sh->tslots = ts == 1 ? 0 : ts == 2 ? 1 : 3;
+        sh->full = ts > 1 ? full * cus : mbn * ncp;
+        sh->fchunk = (sh->full + 7) / 8;
+        sh->tchunk = ((mbn * ncp - sh->full) * ts + 7) / 8;
+        sh->workgroups = 8 * (sh->fchunk + sh->tchunk) * nbatch;
+    }
+    if (us) *us = best;
+    return best >= 0 && sh->mbn * ncp < 0x7fffffff && sh->lds <= 160 * 1024 && sh->threads <= 64 * kKQMaxWaves;
 }
 }  // namespace
 
@@ -1620,21 +1596,21 @@ bool gemm3_id_supported(int type) {
            gemm3_supported(type);
 }
 
-bool gemm3_id_shape(const WView & w, int64_t max_units, bool one_slice, G3Shape * sh) {
+bool gemm3_id_shape(const WView & w, int64_t max_units, bool one_slice, G3Shape * sh, bool pair) {
     return max_units > 0 && w.G > 0 && w.ntiles > 0 &&
-           kq_shape_ncp(w, max_units, 1, sh, false, false, one_slice ? kKQOneSlice : -2);
+           kq_shape_ncp(w, max_units, 1, sh, false, false, one_slice ? kKQOneSlice : -2, pair);
 }
 
 hipError_t launch_gemm3_id(int type, const WView & w, const ActBuf & a, const GemmUnit * units, const int32_t * nunits,
                            int64_t max_units, bool one_slice, float * dst, int64_t dst_span, hipStream_t s,
-                           const KTime * kt, const float * gsrc, int glu) {
+                           const KTime * kt, const uint8_t * up, int glu) {
     G3Shape sh;
     if (!gemm3_id_supported(type) || a.vdt != QMM_TYPE_Q8_K || !a.bsp || !units || !nunits || a.ldk != w.G * 256 ||
         dst_span <= 0 || dst_span >= ((int64_t)1 << 30) ||
-        (glu >= 0) != (gsrc != nullptr) ||
+        (glu >= 0) != (up != nullptr) ||
         (glu != -1 && glu != QMM_GLU_REGLU && glu != QMM_GLU_GEGLU && glu != QMM_GLU_SWIGLU &&
          glu != QMM_GLU_GEGLU_ERF && glu != QMM_GLU_GEGLU_QUICK) ||
-        !gemm3_id_shape(w, max_units, one_slice, &sh) || a.ncols * a.ldk >= ((int64_t)1 << 31) ||
+        !gemm3_id_shape(w, max_units, one_slice, &sh, up != nullptr) || a.ncols * a.ldk >= ((int64_t)1 << 31) ||
         w.G * a.ldT * 16 >= ((int64_t)1 << 31) || a.ldT < a.ncols)
         return hipErrorInvalidValue;
     KQParams q{};
@@ -1659,25 +1635,25 @@ hipError_t launch_gemm3_id(int type, const WView & w, const ActBuf & a, const Ge
     q.ldk = a.ldk;
     q.ldT = a.ldT;
     q.ncols = a.ncols;
-    q.gsrc = gsrc;
+    q.up = up;
     q.glu = glu;
     q.dspan = dst_span;
     const dim3 g((unsigned)(8 * q.fchunk), 1u), b(sh.threads);
     switch (type) {
-        case QMM_TYPE_Q4_K: return launch_kq_u<true>(q, sh, g, b, s, kt);
-        case QMM_TYPE_Q6_K: return launch_q6k_u<true>(q, sh, g, b, s, kt);
-        case QMM_TYPE_Q5_K: return launch_sbs_u<QMM_TYPE_Q5_K, true>(q, sh, g, b, s, kt);
-        case QMM_TYPE_IQ4_XS: return launch_sbs_u<QMM_TYPE_IQ4_XS, true>(q, sh, g, b, s, kt);
+        case QMM_TYPE_Q4_K: return launch_t<QMM_TYPE_Q4_K, true>(q, sh, g, b, s, kt);
+        case QMM_TYPE_Q6_K: return launch_t<QMM_TYPE_Q6_K, true>(q, sh, g, b, s, kt);
+        case QMM_TYPE_Q5_K: return launch_t<QMM_TYPE_Q5_K, true>(q, sh, g, b, s, kt);
+        case QMM_TYPE_IQ4_XS: return launch_t<QMM_TYPE_IQ4_XS, true>(q, sh, g, b, s, kt);
         default: return hipErrorInvalidValue;
     }
 }
 
 // Launch shape of both kernels (kq_shape): U row-half waves per K slice x KS slices.
-bool gemm3_shape(int type, const WView & w, int64_t N, int64_t nbatch, G3Shape * sh) {
+bool gemm3_shape(int type, const WView & w, int64_t N, int64_t nbatch, G3Shape * sh, bool pair, double * us) {
     if (!gemm3_supported(type) || N <= 0 || nbatch <= 0 || nbatch > 65535 || w.G <= 0 || w.ntiles <= 0) return false;
     // (the K-quant frame's launch rule for the super-block types; the block types' for the rest)
     const bool kframe = type == QMM_TYPE_Q4_K || type == QMM_TYPE_Q6_K || type == QMM_TYPE_Q5_K || type == QMM_TYPE_IQ4_XS;
-    return kq_shape(w, N, nbatch, sh, !kframe);
+    return pair ? kq_pair_shape(w, N, nbatch, sh, !kframe, us) : kq_shape(w, N, nbatch, sh, !kframe);
 }
 
 size_t gemm3_tree_words(const G3Shape & sh) {
@@ -1685,13 +1661,15 @@ size_t gemm3_tree_words(const G3Shape & sh) {
 }
 
 hipError_t launch_gemm3(int type, const WView & w, const TiledAct & a, int64_t nbatch, const GemmBatch & bt,
-                        float * dst, hipStream_t s, const KTime * kt, uint32_t * tree) {
+                        float * dst, hipStream_t s, const KTime * kt, uint32_t * tree, const uint8_t * up, int glu) {
     G3Shape sh;
-    if (!gemm3_shape(type, w, a.N, nbatch, &sh) || !a.A || !a.D || a.nblk != w.G * 8 || a.ntb != (a.N + 31) / 32 ||
+    if ((glu >= 0) != (up != nullptr) || !gemm3_shape(type, w, a.N, nbatch, &sh, up != nullptr) || !a.A || !a.D || a.nblk != w.G * 8 || a.ntb != (a.N + 31) / 32 ||
         a.ntiles != a.ntb * nbatch || a.vdt != vec_dot_type(type))
         return hipErrorInvalidValue;
     if ((type == QMM_TYPE_Q4_K || type == QMM_TYPE_Q5_K) && !a.S) return hipErrorInvalidValue;
     KQParams q{};
+    q.up = up;
+    q.glu = glu;
     q.w = w;
     q.tA = a.A;
     q.tD = a.D;
@@ -1722,13 +1700,13 @@ hipError_t launch_gemm3(int type, const WView & w, const TiledAct & a, int64_t n
     }
     const dim3 g((unsigned)(8 * (q.fchunk + q.tchunk)), (unsigned)nbatch), b(sh.threads);
     switch (type) {
-        case QMM_TYPE_Q4_K: return launch_kq_u<false>(q, sh, g, b, s, kt);
-        case QMM_TYPE_Q6_K: return launch_q6k_u<false>(q, sh, g, b, s, kt);
-        case QMM_TYPE_Q5_K: return launch_sbs_u<QMM_TYPE_Q5_K, false>(q, sh, g, b, s, kt);
-        case QMM_TYPE_IQ4_XS: return launch_sbs_u<QMM_TYPE_IQ4_XS, false>(q, sh, g, b, s, kt);
-        case QMM_TYPE_Q4_0: return launch_blk_u<QMM_TYPE_Q4_0>(q, sh, g, b, s, kt);
-        case QMM_TYPE_Q8_0: return launch_blk_u<QMM_TYPE_Q8_0>(q, sh, g, b, s, kt);
-        case QMM_TYPE_IQ4_NL: return launch_blk_u<QMM_TYPE_IQ4_NL>(q, sh, g, b, s, kt);
+        case QMM_TYPE_Q4_K: return launch_t<QMM_TYPE_Q4_K, false>(q, sh, g, b, s, kt);
+        case QMM_TYPE_Q6_K: return launch_t<QMM_TYPE_Q6_K, false>(q, sh, g, b, s, kt);
+        case QMM_TYPE_Q5_K: return launch_t<QMM_TYPE_Q5_K, false>(q, sh, g, b, s, kt);
+        case QMM_TYPE_IQ4_XS: return launch_t<QMM_TYPE_IQ4_XS, false>(q, sh, g, b, s, kt);
+        case QMM_TYPE_Q4_0: return launch_t<QMM_TYPE_Q4_0, false>(q, sh, g, b, s, kt);
+        case QMM_TYPE_Q8_0: return launch_t<QMM_TYPE_Q8_0, false>(q, sh, g, b, s, kt);
+        case QMM_TYPE_IQ4_NL: return launch_t<QMM_TYPE_IQ4_NL, false>(q, sh, g, b, s, kt);
         default: return hipErrorInvalidValue;
     }
 }

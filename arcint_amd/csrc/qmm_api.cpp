@@ -296,6 +296,20 @@ int ensure_tree(qmm_ctx * ctx, size_t words) {
     return QMM_OK;
 }
 
+// the tree slots of a streaming GEMM launch's tail pieces: nullptr (the blocks run whole) when it
+// has none, or under a capture that would have to grow them
+int gemm3_tree(qmm_ctx * ctx, const G3Shape & g3, uint32_t ** tree) {
+    *tree = nullptr;
+    const size_t tw = gemm3_tree_words(g3);
+    if (!tw) return QMM_OK;
+    if (!ctx->capturing) {
+        const int rc = ensure_tree(ctx, tw);
+        if (rc) return rc;
+    }
+    if (ctx->tree_words >= tw) *tree = ctx->tree;
+    return QMM_OK;
+}
+
 F32Cols f32_cols(const qmm_tensor * t) {
     F32Cols c;
     c.base = (const char *)t->buffer->ptr + t->offs;
@@ -899,6 +913,21 @@ static bool use_gemm_for(int type, const WView & w, int64_t N, int64_t nbatch) {
     return waves >= 512 && passes >= 2 && passes * bytes >= 90e6;
 }
 
+// A gate/up pair on the GEMM (one launch of both products): past one pass of the GEMV, when its
+// estimated time is below that of the GEMV's passes (32 columns each on the MFMA GEMV, 8 on v_dot4):
+// both images streamed once a pass at 2.7 MB a us, 1.3 us a pass beside that, and the GLU launch's 3
+// us more.  Measured (op us, GEMV / GEMM): Q6_K 11008 x 4096 at N = 77 84 / 43, at 203 162 / 73; Q8_0
+// 2048 x 1024 at 40 11.9 / 15.4, at 128 17.4 / 16.0; Q4_K 17408 x 5120 at 40 (two products) 83 / 46.
+static bool use_gemm_pair(int type, const WView & w, int64_t N, int64_t nbatch, G3Shape * sh) {
+    if (N < gemm_min_cols(type)) return false;
+    double us = 0;
+    if (!gemm3_shape(type, w, N, nbatch, sh, true, &us)) return false;
+    if (getenv("QMM_GEMM_MIN_COLS") || nbatch > 1) return nbatch == 1 || use_gemm_for(type, w, N, nbatch);
+    const int64_t per = gemv_mma_supported(type) ? kMmaMaxCols : 8;
+    const double bytes = 2.0 * (double)(w.ntiles * w.G) * (double)w.tg;
+    return us + 2.0 < 3.0 + (double)((N + per - 1) / per) * (1.3 + bytes / 2.7e6);
+}
+
 // columns per GEMV task: up to 32 on the MFMA kernel (the rows of its A operand), 8 on v_dot4,
 // spread evenly over the fewest weight passes
 static int gemv_task_cols(int type, int64_t N) {
@@ -1161,11 +1190,7 @@ static int mul_mat_launch(qmm_ctx * ctx, const qmm_tensor * src0, const qmm_tens
         // the blocks past a whole number per CU in K pieces meeting in tree slots (grown outside
         // captures only; without them, and in qmm_mul_mat_noalloc, the blocks run whole)
         uint32_t * tree = nullptr;
-        const size_t tw = gemm3_tree_words(g3);
-        if (tw && !fixed) {
-            if (!ctx->capturing && (rc = ensure_tree(ctx, tw))) return rc;
-            if (ctx->tree_words >= tw) tree = ctx->tree;
-        }
+        if (!fixed && (rc = gemm3_tree(ctx, g3, &tree))) return rc;
         if (!fixed && (rc = ktime_pair(ctx, &kt, &ktp))) return rc;
         QMM_HIP(ctx, launch_gemm3(src0->type, w, ta, nbatch, bt, d, ctx->stream, ktp, tree));
         return ktime_done(ctx);
@@ -1487,23 +1512,17 @@ int qmm_mul_mat_id_glu(qmm_ctx * ctx, const qmm_tensor * gate, const qmm_tensor 
         return rc;
     }
     if (use_moe_gemm(gate->type, wg, npairs, n_as, true) && id_dst_span(dst) <= kMaxIdSpan) {
-        // the grouped GEMM: one route and quantization for both products; gate into the scratch
-        // at dst's offsets, then up with act(gate) * up applied at its stores
+        // the grouped GEMM: one route and quantization, one launch for both products and the GLU
         const int64_t dnb1 = (int64_t)(dst->nb[1] / 4), dnb2 = (int64_t)(dst->nb[2] / 4);
-        const int64_t span = id_dst_span(dst);
-        if ((rc = ensure(ctx, &ctx->glu, &ctx->glu_cap, (size_t)span * sizeof(float)))) return rc;
         const int64_t max_units = route_max_units(npairs, n_as);
         GemmUnit * units;
         int32_t * nunits;
         PendingRoute pr;
         if ((rc = route_units(ctx, ids, src1->ne[1], n_as, dnb1, dnb2, max_units, &units, &nunits, &pr))) return rc;
         if ((rc = quantize_src1(ctx, gate->type, src1, false, &a, nullptr, &pr))) return rc;
-        float * g = (float *)ctx->glu;
         float * d = (float *)((uint8_t *)dst->buffer->ptr + dst->offs);
-        const bool one = moe_one_slice(wg, npairs, n_as);
-        QMM_HIP(ctx, launch_gemm3_id(gate->type, wg, a, units, nunits, max_units, one, g, span, ctx->stream));
-        QMM_HIP(ctx, launch_gemm3_id(up->type, wu, a, units, nunits, max_units, one, d, span, ctx->stream, nullptr, g,
-                                     glu_op));
+        QMM_HIP(ctx, launch_gemm3_id(gate->type, wg, a, units, nunits, max_units, moe_one_slice(wg, npairs, n_as), d,
+                                     id_dst_span(dst), ctx->stream, nullptr, wu.base, glu_op));
         ctx->path = "glu-gemm-id-stream";
         return QMM_OK;
     }
@@ -1955,6 +1974,25 @@ int qmm_mul_mat_glu(qmm_ctx * ctx, const qmm_tensor * gate, const qmm_tensor * u
             ctx->path = "glu-fused-gemv-fq";
             return frc;
         }
+        // the streaming GEMM: gate and up waves side by side in each work-group, the GLU where their
+        // sums meet
+        const int64_t nbatch = dn.ne12 * dn.ne13;
+        G3Shape g3;
+        if (use_gemm_pair(gate->type, wg, src1->ne[1], nbatch, &g3)) {
+            TiledAct ta;
+            int rc = quantize_src1_tiled(ctx, gate->type, src1, wg.G, &ta);
+            if (rc) return rc;
+            const GemmBatch bt{ dn.ne12, dn.r2, dn.r3, dn.ne02, dn.d_nb1, dn.d_nb2, dn.d_nb3 };
+            uint32_t * tree = nullptr;
+            if ((rc = gemm3_tree(ctx, g3, &tree))) return rc;
+            KTime kt;
+            const KTime * ktp;
+            if ((rc = ktime_pair(ctx, &kt, &ktp))) return rc;
+            ctx->path = "glu-gemm-stream";
+            QMM_HIP(ctx, launch_gemm3(gate->type, wg, ta, nbatch, bt, (float *)((uint8_t *)dst->buffer->ptr + dst->offs),
+                                      ctx->stream, ktp, tree, wu.base, glu_op));
+            return ktime_done(ctx);
+        }
     }
     const int64_t M = gate->ne[1], N = src1->ne[1], ne12 = src1->ne[2], nb = src1->ne[2] * src1->ne[3];
     const size_t half = (size_t)(M * N * nb);
@@ -1964,7 +2002,9 @@ int qmm_mul_mat_glu(qmm_ctx * ctx, const qmm_tensor * gate, const qmm_tensor * u
     const int type = gate->type;
     const int nc = gemv_task_cols(type, N);
     GemvPlan plan;
-    const bool fused = up->type == type && nb == 1 && !use_gemm_for(type, wg, N, nb) &&
+    // (a pair of one type and batch that did not take the streaming GEMM above is the GEMV's, unless
+    // that GEMM is switched off)
+    const bool fused = up->type == type && nb == 1 && (gemm3_supported(type) || !use_gemm_for(type, wg, N, nb)) &&
                        gemv_plan(type, wg, nc, (N + nc - 1) / nc * 2, true, nc >= gemv_mma_min_cols(), &plan);
     if (fused) {
         GemvDense dn;

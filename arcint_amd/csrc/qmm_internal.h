@@ -400,26 +400,29 @@ struct G3Shape {
     int ts, pk, tslots;
     int64_t fchunk, tchunk;        // per XCD: whole blocks, tail pieces
 };
-bool gemm3_shape(int type, const WView & w, int64_t N, int64_t nbatch, G3Shape * sh);
+// pair: a gate/up pair in one launch (see launch_gemm3), us its estimated kernel time
+bool gemm3_shape(int type, const WView & w, int64_t N, int64_t nbatch, G3Shape * sh, bool pair = false,
+                 double * us = nullptr);
 // tree words the tail pieces of that launch meet in (0: no pieces)
 size_t gemm3_tree_words(const G3Shape & sh);
 // Grouped MoE GEMM (MUL_MAT_ID with many pairs per expert): the route's 64-column units
 // (*nunits of at most max_units) of one expert each, activations gathered from the route's q8_K
 // quantization a; unit pairs with mat < 0 get zero rows.  Q4_K, Q6_K, Q5_K and IQ4_XS.
 // dst_span: the floats from dst to one past its last element (below 2^30: the stores take
-// 32-bit byte offsets).  With glu >= 0 (QMM_GLU_*) this is the up product of a gate/up pair:
-// each stored value is act(gsrc[o]) * up at its dst offset o, gsrc the gate product's rows at
-// the same offsets (zero rows stay zero).  one_slice: 4-wave one-slice blocks, three a CU
+// 32-bit byte offsets).  With glu >= 0 (QMM_GLU_*) the launch is a gate/up pair: w the gate stack,
+// up the image of the up stack (same shape and type), dst = act(gate) * up (zero rows stay zero).  one_slice: 4-wave one-slice blocks, three a CU
 // (mostly full units, a block per CU or more), else the launch rule's shape.
 bool gemm3_id_supported(int type);
-bool gemm3_id_shape(const WView & w, int64_t max_units, bool one_slice, G3Shape * sh);
+bool gemm3_id_shape(const WView & w, int64_t max_units, bool one_slice, G3Shape * sh, bool pair = false);
 hipError_t launch_gemm3_id(int type, const WView & w, const ActBuf & a, const GemmUnit * units, const int32_t * nunits,
                            int64_t max_units, bool one_slice, float * dst, int64_t dst_span, hipStream_t s,
-                           const KTime * kt = nullptr, const float * gsrc = nullptr, int glu = -1);
+                           const KTime * kt = nullptr, const uint8_t * up = nullptr, int glu = -1);
 // tree: gemm3_tree_words(shape) words of tree slots, each kTreeEmpty (left so), or nullptr: then
-// the tail blocks run whole
+// the tail blocks run whole.  glu >= 0 (QMM_GLU_*): a gate/up pair in one launch, w the gate's
+// image and up the up matrix's (same shape and type): dst = act(gate) * up
 hipError_t launch_gemm3(int type, const WView & w, const TiledAct & a, int64_t nbatch, const GemmBatch & bt,
-                        float * dst, hipStream_t s, const KTime * kt = nullptr, uint32_t * tree = nullptr);
+                        float * dst, hipStream_t s, const KTime * kt = nullptr, uint32_t * tree = nullptr,
+                        const uint8_t * up = nullptr, int glu = -1);
 
 // K slices the GEMM splits this product into; above 1 the slices add their
 // partial sums to dst with atomics, so dst must be zeroed first.

@@ -213,7 +213,8 @@ int    qmm_mul_mat_id(qmm_ctx * ctx, const qmm_tensor * src0, const qmm_tensor *
  * matches (P01:65; ggml-opencl.cpp:9836-9878 by the reference's audit,
  * docs/campaigns/research-concept-mining/ipex-llm/audit.md:83-87).  One activation
  * quantization serves both; at GEMV widths with one batch and one weight type both matrices
- * stream in one launch.  Within MUL_MAT's tolerance of the unfused chain. */
+ * stream in one launch, as they do on the streaming GEMM (gate and up waves side by side in each
+ * work-group).  Within MUL_MAT's tolerance of the unfused chain. */
 int    qmm_mul_mat_glu(qmm_ctx * ctx, const qmm_tensor * gate, const qmm_tensor * up, const qmm_tensor * src1,
                        const qmm_tensor * dst, int32_t glu_op);
 /* The MoE form: dst = act(MUL_MAT_ID(gate, src1, ids)) * MUL_MAT_ID(up, src1, ids), gate and
@@ -221,8 +222,7 @@ int    qmm_mul_mat_glu(qmm_ctx * ctx, const qmm_tensor * gate, const qmm_tensor 
  * Replaces MUL_MAT_ID, MUL_MAT_ID, GLU (the reference's MUL_MAT_ID / GLU fuse, by its audit
  * docs/campaigns/research-concept-mining/ipex-llm/audit.md:83-87): one quantization, one
  * route, one GEMV launch over both stacks; experts averaging the grouped GEMM's pair count
- * (QMM_MOE_GEMM_MIN) take it twice, the GLU applied at the up product's stores.  Invalid ids
- * give zero rows. */
+ * (QMM_MOE_GEMM_MIN) take one launch of that over both.  Invalid ids give zero rows. */
 int    qmm_mul_mat_id_glu(qmm_ctx * ctx, const qmm_tensor * gate, const qmm_tensor * up, const qmm_tensor * src1,
                           const qmm_tensor * ids, const qmm_tensor * dst, int32_t glu_op);
 /* qmm_mul_mat with nothing allocated: no reference counterpart; for callers that cannot
@@ -360,10 +360,11 @@ int64_t qmm_downgrades(qmm_ctx * ctx, char * buf, size_t buf_len);
  * + the streaming int8 MFMA GEMM), "gemm-mfma" (pre-pass + the shared-tile int8 MFMA GEMM).
  * MUL_MAT_ID: "gemv-id-fq" (one launch, each (slot, token) pair read from ids), "gemv-id" /
  * "gemv-id-mfma" (route + expert tasks on either GEMV), "gemm-id-stream" (route + the grouped
- * streaming GEMM).  qmm_mul_mat_glu: "glu-fused-gemv-fq", "glu-fused-gemv", "glu-fused-gemv-mfma"
- * (gate and up in one launch) or "glu-" + the MUL_MAT path (two products and a GLU kernel).
+ * streaming GEMM).  qmm_mul_mat_glu: "glu-fused-gemv-fq", "glu-fused-gemv", "glu-fused-gemv-mfma",
+ * "glu-gemm-stream" (gate and up in one launch) or "glu-" + the MUL_MAT path (two products and a GLU
+ * kernel: mixed types, batches on the GEMV).
  * qmm_mul_mat_id_glu: "glu-gemv-id-fq", "glu-gemv-id", "glu-gemv-id-mfma", "glu-gemm-id-stream"
- * (route + the grouped GEMM for gate, then for up with the GLU at its stores).  The router and
+ * (route + one grouped GEMM launch over both stacks).  The router and
  * the combine: "moe-topk", "moe-combine"; qmm_moe_ffn: "moe-ffn-fq" (below 16 tokens),
  * "moe-ffn-route". */
 const char * qmm_last_path(qmm_ctx * ctx);
