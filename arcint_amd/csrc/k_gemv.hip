@@ -1381,8 +1381,24 @@ __device__ __forceinline__ void quant_slot(float (&v)[4], uint8_t * slot, int la
 // A work-group is W waves on one 64-row tile of one task, wave w streaming groups
 // [w spw, w spw + spw) (dot4_stages with one K slice).  LDS: the waves' slots [W][spw][NC], then,
 // after the stream, the waves' sums [W][NV][64].
-template <int TYPE, int NC, bool ROUTE = false>
+// MODE: what the launch is, a template argument so that a kernel holds its own steps only (with the
+// modes as run-time branches every launch paid for fetching past the others': a one-column product
+// 0.5-0.9 us of its 5-16, see k_gemv_fq1)
+enum FqMode {
+    kFqDense,      // dense tasks
+    kFqDenseGlu,   // dense gate/up pairs
+    kFqIds,        // MUL_MAT_ID pairs
+    kFqIdsGlu,     // MUL_MAT_ID gate/up pairs
+    kFqIdsRoute,   // the same, ranking the router's logits itself
+    kFqCombTree,   // MoE down, slots met in the exchange tree
+    kFqCombSlots,  // MoE down, slots as waves
+};
+template <int TYPE, int NC, int MODE>
 __global__ __launch_bounds__(1024) void k_gemv_fq(FqParams p) {
+    constexpr bool IDS = MODE >= kFqIds, ROUTE = MODE == kFqIdsRoute, COMB = MODE == kFqCombTree;
+    constexpr bool glu = MODE == kFqDenseGlu || MODE == kFqIdsGlu || MODE == kFqIdsRoute;
+    // combine mode 2 (MoE down, slots as waves): wave w is slot w of the token over the whole K
+    constexpr bool slotw = MODE == kFqCombSlots;
     using T = GV<TYPE>;
     constexpr int NL = T::NL, NST = T::NST;
     constexpr int VDT = (TYPE == QMM_TYPE_Q4_0 || TYPE == QMM_TYPE_Q8_0 || TYPE == QMM_TYPE_IQ4_NL) ? QMM_TYPE_Q8_0
@@ -1395,13 +1411,11 @@ __global__ __launch_bounds__(1024) void k_gemv_fq(FqParams p) {
     // the grid is the position: (tiles, slots, tokens) for MUL_MAT_ID pairs, pair p = t n_used + i;
     // (tiles, tasks, K slices) for dense products
     const uint32_t tile = blockIdx.x, task = blockIdx.y;
-    const int ks = p.ids ? 0 : (int)blockIdx.z;
+    const int ks = IDS ? 0 : (int)blockIdx.z;
     int mat, nc;
     int64_t colv[NC], doffv[NC];
     bool shared = false, skip = false;
     const int G = (int)p.w.G;
-    // combine mode 2 (MoE down, slots as waves): wave w is slot w of the token over the whole K
-    const bool slotw = p.comb == 2;                               // uniform
     int ga, S;
     dot4_stages(ks, slotw ? 1 : p.W, slotw ? 0 : wave, p.spw, G, NST, ga, S);
     // the wave's activation groups, quantized into its slots [group][column]
@@ -1420,7 +1434,7 @@ __global__ __launch_bounds__(1024) void k_gemv_fq(FqParams p) {
         }
         xq = true;
     };
-    if (p.ids) {
+    if constexpr (IDS) {
         const int64_t t = blockIdx.z, i = slotw ? wave : blockIdx.y;
         shared = i >= p.n_used;                                   // uniform (over the wave): the shared expert's slot
         nc = 1;
@@ -1454,7 +1468,7 @@ __global__ __launch_bounds__(1024) void k_gemv_fq(FqParams p) {
         const int64_t doff = t * p.dnb2 + i * p.dnb1;
         if (e < 0 || e >= p.n_as) {                                // uniform: a zero row
             if ((slotw || wave == 0) && e >= p.n_as && tile == 0 && lane == 0) *p.bad_id = 1;
-            if (!p.comb) {
+            if constexpr (!COMB && !slotw) {
                 if (wave == 0) {
                     const int64_t row = (int64_t)tile * kTileRows + lane;
                     if (row < p.w.M) p.dst[doff + row] = 0.0f;
@@ -1481,8 +1495,10 @@ __global__ __launch_bounds__(1024) void k_gemv_fq(FqParams p) {
         }
     }
     nc = __builtin_amdgcn_readfirstlane(nc);
+    // (not a constant to the compiler: with the dots' column branches gone it gathers all of a stage's
+    // activation reads ahead of them, and spills 30-60 of 128 registers)
+    asm volatile("" : "+s"(nc));
     if (skip) S = 0;                                              // (a zero row: no stages, no groups)
-    const bool glu = p.glu >= 0;                                  // uniform
     const int ST = glu ? 2 * S : S;                               // gate stages, then up stages
     WView w1 = p.w, w2 = p.w;
     if (shared) w1.base = p.sh_base;
@@ -1553,7 +1569,7 @@ __global__ __launch_bounds__(1024) void k_gemv_fq(FqParams p) {
         }
     }
     const int64_t row = (int64_t)tile * kTileRows + lane;
-    if (slotw) {                                                  // uniform (MoE down, one column)
+    if constexpr (slotw) {                                        // (MoE down, one column)
         // each slot's row times its weight (rounded, as the graph's MUL), then the token's rows
         // added slot by slot, the routed ones in order and the gated shared expert last: the
         // graph's chain of ADDs
@@ -1581,7 +1597,7 @@ __global__ __launch_bounds__(1024) void k_gemv_fq(FqParams p) {
         __syncthreads();                                          // every wave is done with the slots
 #pragma unroll
         for (int j = 0; j < NC; ++j) red[(wave * NV + j) * 64 + lane] = acc[j];
-        if (glu) {
+        if constexpr (glu) {
 #pragma unroll
             for (int j = 0; j < NC; ++j) red[(wave * NV + NC + j) * 64 + lane] = accu[j];
         }
@@ -1608,12 +1624,12 @@ __global__ __launch_bounds__(1024) void k_gemv_fq(FqParams p) {
     bool alive[NC];
 #pragma unroll
     for (int j = 0; j < NC; ++j) alive[j] = true;
-    if (p.KS > 1) {                                               // uniform (dense)
+    if (!IDS && p.KS > 1) {                                       // uniform
         uint32_t * nodes = p.tree + ((size_t)task * (size_t)p.w.ntiles + tile) * (2 * (size_t)p.KS * NC * 64) * (glu ? 2 : 1);
-        if (glu) tree_add_pairs<NC>(reinterpret_cast<uint64_t *>(nodes), ks, p.KS, nc, tot, totu, alive, lane);
+        if constexpr (glu) tree_add_pairs<NC>(reinterpret_cast<uint64_t *>(nodes), ks, p.KS, nc, tot, totu, alive, lane);
         else tree_add<NC>(nodes, ks, p.KS, nc, tot, alive, lane);
     }
-    if (p.comb) {                                                 // uniform (MoE down, one column)
+    if constexpr (COMB) {                                         // (MoE down, one column)
         // the slot's row times its weight (each product rounded, as the graph's MUL), then the
         // token's slots added in the tree; every slot of every tile takes part, so each node
         // sees its two exchanges and the launch leaves the slots empty
@@ -1633,6 +1649,82 @@ __global__ __launch_bounds__(1024) void k_gemv_fq(FqParams p) {
 #pragma unroll
     for (int j = 0; j < NC; ++j)
         if (j < nc && alive[j]) p.dst[doffv[j] + row] = glu ? glu_apply(p.glu, tot[j], totu[j]) : tot[j];
+}
+
+// ---- one-column dense products, one launch for up to kFq1Max of them --------------------------
+// k_gemv_fq's split form (one group a wave, W waves a work-group, KS work-groups per tile met in the
+// exchange tree) with nothing else in the kernel, for a list of independent products: work-group
+// (x, y) is tile x - start[i] of product i, K slice y.  A decode step's projections are a few tens of MB
+// in all, and each launch ramps up and drains for ~4 us, which the next one waits for: Q5_K 12288, 1024
+// and 1024 x 5120 and 5120 x 6144 one after the other 29.2 us (26.8 on this kernel), in one launch 15.1.  Sums meet in the
+// same order as k_gemv_fq's (the same bits).
+struct Fq1Params {
+    Fq1Mat m[kFq1Max];
+    uint32_t start[kFq1Max];     // first tile index (x) of each product, 0xffffffff past the last
+    const uint8_t * sink;
+    int W;
+};
+
+template <int TYPE, int MAXM>
+__global__ __launch_bounds__(512) void k_gemv_fq1(Fq1Params p) {
+    using T = GV<TYPE>;
+    constexpr int VDT = (TYPE == QMM_TYPE_Q4_0 || TYPE == QMM_TYPE_Q8_0 || TYPE == QMM_TYPE_IQ4_NL) ? QMM_TYPE_Q8_0
+                                                                                                     : QMM_TYPE_Q8_K;
+    static_assert(T::kReadEnd <= tile_group_bytes(TYPE) && tile_group_bytes(TYPE) <= (int)kSinkBytes,
+                  "a stage reads inside one tile-group, which fits in the sink");
+    extern __shared__ __align__(16) uint8_t sm[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ks = (int)blockIdx.y;
+    uint32_t tile = blockIdx.x;
+    int i = 0;
+    if constexpr (MAXM > 1) {
+#pragma unroll
+        for (int k = 1; k < MAXM; ++k) i += tile >= p.start[k] ? 1 : 0;
+        tile -= p.start[i];
+    }
+    const Fq1Mat & m = p.m[i];
+    if (MAXM > 1 && ks >= m.KS) return;                           // uniform: a shorter K than the longest's
+    const int ga = ks * p.W + wave;                               // the wave's group
+    const bool in = ga < m.G;                                     // uniform over the wave
+    // the activations are requested ahead of the weights (both without a branch: a wave past K
+    // reads column 0's start and the sink)
+    const int64_t k0 = (int64_t)ga * 256 + 4 * lane;
+    const bool kin = k0 < m.K;
+    const float * x = m.x + (kin ? k0 : 0);
+    float xv[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float t = x[e];
+        xv[e] = kin ? t : 0.0f;
+    }
+    const uint8_t * tg = in ? m.base + ((size_t)tile * (size_t)m.G + (size_t)ga) * (size_t)tile_group_bytes(TYPE) : p.sink;
+    uint4 B[T::NL], B1[T::NL];
+    T::load(B, tg, 0, lane);
+    if constexpr (T::NST == 2) T::load(B1, tg, 1, lane);
+    uint8_t * const slot = sm + wave * kFqSlot;
+    quant_slot<VDT>(xv, slot, lane);
+    __builtin_amdgcn_wave_barrier();
+    XL<1> xl;
+    xl.c[0] = reinterpret_cast<const int8_t *>(slot);
+    xl.d[0] = reinterpret_cast<const float *>(slot + 256);
+    xl.s[0] = reinterpret_cast<const int16_t *>(slot + 288);
+    float acc[1] = { 0.0f };
+    int state[1] = { 0 };
+    if (in) {
+        T::dot(B, 0, xl, 1, acc, state);
+        if constexpr (T::NST == 2) T::dot(B1, 1, xl, 1, acc, state);
+    }
+    float * red = reinterpret_cast<float *>(sm + p.W * kFqSlot);
+    red[wave * 64 + lane] = acc[0];
+    __syncthreads();
+    if (wave != 0) return;
+    float tot[1] = { red[lane] };
+    for (int w = 1; w < p.W; ++w) tot[0] += red[w * 64 + lane];
+    bool alive[1] = { true };
+    if (m.KS > 1) tree_add<1>(m.tree + (size_t)tile * (2 * (size_t)m.KS * 64), ks, m.KS, 1, tot, alive, lane);
+    const int64_t row = (int64_t)tile * kTileRows + lane;
+    if (row < m.M && alive[0]) m.dst[row] = tot[0];
 }
 
 }  // namespace
@@ -1680,6 +1772,50 @@ bool gemv_fused_slot_plan(int type, const WView & w, int64_t nslots, int64_t T, 
     pl->KS = 1;
     pl->lds = std::max<int64_t>(nslots * w.G * kFqSlot, nslots * 64 * 4);
     return pl->lds <= 64 * 1024 && T * w.ntiles < 0x7fffffff;
+}
+
+int64_t gemv_fq1_tree_words(const Fq1Mat & m) { return m.KS > 1 ? (m.M + kTileRows - 1) / kTileRows * 2 * m.KS * 64 : 0; }
+
+hipError_t launch_gemv_fq1(int type, const Fq1Mat * m, int n, int W, const void * sink, hipStream_t s, const KTime * kt) {
+    if (n < 1 || n > kFq1Max || W < 1 || W > 8 || !sink) return hipErrorInvalidValue;
+    Fq1Params p{};
+    p.sink = (const uint8_t *)sink;
+    p.W = W;
+    int64_t tiles = 0;
+    int ks = 1;
+    for (int i = 0; i < kFq1Max; ++i) {
+        p.start[i] = 0xffffffffu;
+        if (i >= n) continue;
+        if (!m[i].base || !m[i].x || !m[i].dst || m[i].G < 1 || m[i].M < 1 || m[i].KS != (m[i].G + W - 1) / W ||
+            (m[i].KS > 1 && !m[i].tree) || m[i].KS > 65535)
+            return hipErrorInvalidValue;
+        p.m[i] = m[i];
+        p.start[i] = (uint32_t)tiles;
+        tiles += (m[i].M + kTileRows - 1) / kTileRows;
+        ks = std::max(ks, m[i].KS);
+    }
+    if (tiles >= 0x7fffffff) return hipErrorInvalidValue;
+    const dim3 g((unsigned)tiles, (unsigned)ks), b(64 * W);
+    const uint32_t lds = (uint32_t)(W * (kFqSlot + 256));
+#define QMM_FQ1_K(...)                                                                              \
+    if (kt) hipExtLaunchKernelGGL((__VA_ARGS__), g, b, lds, s, kt->start, kt->stop, 0, p);          \
+    else (__VA_ARGS__)<<<g, b, lds, s>>>(p);                                                        \
+    return hipGetLastError();
+#define QMM_FQ1(T)                                                                                  \
+    if (n == 1) { QMM_FQ1_K(k_gemv_fq1<T, 1>) }                                                     \
+    QMM_FQ1_K(k_gemv_fq1<T, kFq1Max>)
+    switch (type) {
+        case QMM_TYPE_Q4_0: { QMM_FQ1(QMM_TYPE_Q4_0) }
+        case QMM_TYPE_Q8_0: { QMM_FQ1(QMM_TYPE_Q8_0) }
+        case QMM_TYPE_Q4_K: { QMM_FQ1(QMM_TYPE_Q4_K) }
+        case QMM_TYPE_Q5_K: { QMM_FQ1(QMM_TYPE_Q5_K) }
+        case QMM_TYPE_Q6_K: { QMM_FQ1(QMM_TYPE_Q6_K) }
+        case QMM_TYPE_IQ4_XS: { QMM_FQ1(QMM_TYPE_IQ4_XS) }
+        case QMM_TYPE_IQ4_NL: { QMM_FQ1(QMM_TYPE_IQ4_NL) }
+        default: return hipErrorInvalidValue;
+    }
+#undef QMM_FQ1
+#undef QMM_FQ1_K
 }
 
 int64_t gemv_fused_tree_words(const WView & w, const FusedPlan & pl, bool glu) {
@@ -1770,9 +1906,15 @@ hipError_t launch_gemv_fused(int type, const WView & w, const FusedPlan & pl, co
     else __VA_ARGS__<<<g, b, lds, s>>>(p);                                                          \
     return hipGetLastError();
 #define QMM_FQ(T)                                                                                   \
-    if (f.lg) { QMM_FQ_K(k_gemv_fq<T, 1, true>) }                                                   \
-    if (pl.nc == 1) { QMM_FQ_K(k_gemv_fq<T, 1>) }                                                   \
-    QMM_FQ_K(k_gemv_fq<T, 2>)
+    if (f.lg) { QMM_FQ_K((k_gemv_fq<T, 1, kFqIdsRoute>)) }                                          \
+    if (f.comb == 2) { QMM_FQ_K((k_gemv_fq<T, 1, kFqCombSlots>)) }                                  \
+    if (f.comb) { QMM_FQ_K((k_gemv_fq<T, 1, kFqCombTree>)) }                                        \
+    if (f.ids && f.glu >= 0) { QMM_FQ_K((k_gemv_fq<T, 1, kFqIdsGlu>)) }                             \
+    if (f.ids) { QMM_FQ_K((k_gemv_fq<T, 1, kFqIds>)) }                                              \
+    if (f.glu >= 0 && pl.nc == 1) { QMM_FQ_K((k_gemv_fq<T, 1, kFqDenseGlu>)) }                      \
+    if (f.glu >= 0) { QMM_FQ_K((k_gemv_fq<T, 2, kFqDenseGlu>)) }                                    \
+    if (pl.nc == 1) { QMM_FQ_K((k_gemv_fq<T, 1, kFqDense>)) }                                       \
+    QMM_FQ_K((k_gemv_fq<T, 2, kFqDense>))
     switch (type) {
         case QMM_TYPE_Q4_0: { QMM_FQ(QMM_TYPE_Q4_0) }
         case QMM_TYPE_Q8_0: { QMM_FQ(QMM_TYPE_Q8_0) }

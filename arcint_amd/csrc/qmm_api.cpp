@@ -1094,6 +1094,29 @@ int qmm_describe_mul_mat(const qmm_tensor * src0, const qmm_tensor * src1, const
     return QMM_OK;
 }
 
+// A split-form product of one column and batch, one group a wave, takes k_gemv_fq1 (the same sums, and
+// nothing in the kernel beside them: Q4_0 4096 x 4096 4.95 -> 4.28 us, Q6_K 5120 x 17408 15.3-15.8 ->
+// 14.8, IQ4_XS 4096 x 14336 10.3 -> 9.45, Q4_K 17408 x 5120 10.8-11.0 -> 10.6), but for Q6_K images past
+// the 256 MB Infinity Cache: at 75 registers against 100 six of its waves share a SIMD, not four, and
+// their two-stage requests queue up (151936 x 5120, 638 MB: 97.5 us against 95.9; 40000 x 5120, 168 MB,
+// the same; Q4_K of 350 MB 58.0 against 58.6).  QMM_GEMV_FQ1=0: never.
+static bool fq1_for(int type, const WView & w, const FusedPlan & fp) {
+    return fp.nc == 1 && fp.ntasks == 1 && fp.spw == 1 && fp.KS > 1 && fp.W <= 8 && env_or("QMM_GEMV_FQ1", 1) != 0 &&
+           (type != QMM_TYPE_Q6_K || w.ntiles * w.G * (int64_t)w.tg < ((int64_t)256 << 20));
+}
+static Fq1Mat fq1_mat(const qmm_tensor * src1, const WView & w, float * d, int W, uint32_t * tree) {
+    return Fq1Mat{ w.base, (const float *)((const uint8_t *)src1->buffer->ptr + src1->offs), d, tree, w.M, w.K, (int32_t)w.G,
+                   (int32_t)((w.G + W - 1) / W) };
+}
+static int fq1_launch(qmm_ctx * ctx, int type, const Fq1Mat * m, int n, int W) {
+    KTime kt;
+    const KTime * ktp = nullptr;
+    const int rc = ktime_pair(ctx, &kt, &ktp);
+    if (rc) return rc;
+    const hipError_t e = launch_gemv_fq1(type, m, n, W, ctx->sink, ctx->stream, ktp);
+    return e == hipSuccess ? ktime_done(ctx) : fail(ctx, QMM_ERR_DEVICE, "launch_gemv_fq1: %s", hipGetErrorString(e));
+}
+
 // a dense fused launch when the shape suits it (false: not taken, nothing enqueued)
 static bool try_fused_dense(qmm_ctx * ctx, const qmm_tensor * src0, const qmm_tensor * src1, const WView & w,
                             const GemvDense & dn, float * d, const uint8_t * up_base, int glu, bool noalloc, int * rc) {
@@ -1103,6 +1126,11 @@ static bool try_fused_dense(qmm_ctx * ctx, const qmm_tensor * src0, const qmm_te
     if (fp.KS > 1) {
         if ((*rc = ensure_tree(ctx, (size_t)gemv_fused_tree_words(w, fp, glu >= 0)))) return true;
         f.tree = ctx->tree;
+        if (glu < 0 && fq1_for(src0->type, w, fp)) {
+            const Fq1Mat m = fq1_mat(src1, w, d, fp.W, ctx->tree);
+            *rc = fq1_launch(ctx, src0->type, &m, 1, fp.W);
+            return true;
+        }
     }
     f.x = f32_cols(src1);
     f.K = src1->ne[0];

@@ -333,6 +333,22 @@ int gemv_fused_waves_target();
 hipError_t launch_gemv_fused(int type, const WView & w, const FusedPlan & plan, const FusedGemv & f, float * dst,
                              const void * sink, hipStream_t s, const KTime * kt = nullptr);
 
+// One-column dense products without batches, up to kFq1Max of one type in one launch (k_gemv_fq1): each
+// its image, its activation column and its dst column (M floats), KS = ceil(G / W) K slices of W waves;
+// tree: gemv_fq1_tree_words words of slots of its own, each kTreeEmpty (left so), when KS > 1.
+constexpr int kFq1Max = 8;
+struct Fq1Mat {
+    const uint8_t * base;
+    const float * x;
+    float * dst;
+    uint32_t * tree;
+    int64_t M, K;
+    int32_t G, KS;
+};
+int64_t gemv_fq1_tree_words(const Fq1Mat & m);
+hipError_t launch_gemv_fq1(int type, const Fq1Mat * m, int n, int W, const void * sink, hipStream_t s,
+                           const KTime * kt = nullptr);
+
 // Prefill GEMM (int8 MFMA, all five types): for every batch b < nbatch,
 // dst[doff(b) + n * d_nb1 + m] = W(mat(b)) row m . activation column
 // col0(b) + n, for n < N, m < M.  Activations come from the pre-pass with
