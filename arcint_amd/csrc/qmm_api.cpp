@@ -275,6 +275,8 @@ int ensure(qmm_ctx * ctx, void ** p, size_t * cap, size_t need) {
     return QMM_OK;
 }
 
+// the slots' first size: 4 MB, what a decode step's projections of ~350 MB of weights meet in
+constexpr size_t kTreeMinWords = (size_t)1 << 20;
 // tree slots for a split fused GEMV: grown outside captures only, each new allocation filled
 // with kTreeEmpty on the stream ahead of its first use
 int ensure_tree(qmm_ctx * ctx, size_t words) {
@@ -289,7 +291,7 @@ int ensure_tree(qmm_ctx * ctx, size_t words) {
         ctx->tree_words = 0;
         ctx->scratch_gen++;
     }
-    const size_t n = std::max(words, ctx->tree_words * 3 / 2);
+    const size_t n = std::max({ words, ctx->tree_words * 3 / 2, kTreeMinWords });
     QMM_HIP(ctx, hipMalloc((void **)&ctx->tree, n * 4));
     QMM_HIP(ctx, hipMemsetD32Async((hipDeviceptr_t)ctx->tree, (int)kTreeEmpty, n, ctx->stream));
     ctx->tree_words = n;
@@ -2184,27 +2186,92 @@ int qmm_internal_gemv_extent(int32_t type, const int64_t ne0[4], int64_t N, int6
     return QMM_OK;
 }
 
+// The run of one-column MUL_MAT nodes from nodes[0] that one k_gemv_fq1 launch takes: one weight type,
+// each on the one-column split or one-slice plan, none reading or writing what another writes.
+// Returns how many (0 or 1: none, run node by node).  A run's slots stay within kTreeMinWords, which
+// every context with slots has, so no run makes the slots grow (and captured graphs void) or, under
+// a capture, need more than a context that ran any split product has.  Kernel timing stamps every
+// op's own kernel, so it takes the nodes one by one.
+static int fq1_run(qmm_ctx * ctx, const qmm_node * nodes, int n_nodes, Fq1Mat * m, int * W) {
+    if (ctx->ktime || env_or("QMM_GEMV_GROUP", 1) == 0 || (ctx->capturing && ctx->tree_words < kTreeMinWords)) return 0;
+    int n = 0;
+    size_t words = 0;
+    for (; n < n_nodes && n < kFq1Max; ++n) {
+        const qmm_node & a = nodes[n];
+        WView w;
+        if (a.op != QMM_OP_MUL_MAT || !mul_mat_ok(a.src0, a.src1, a.dst, true, &w, nullptr, 0)) break;
+        const int type = a.src0->type;
+        if (a.src1->ne[1] != 1 || a.src1->ne[2] * a.src1->ne[3] != 1 || (n && type != nodes[0].src0->type)) break;
+        FusedPlan fp;
+        if (use_gemm_for(type, w, 1, 1) || !fused_dense_plan(type, w, 1, 1, &fp, true) || fp.nc != 1) break;
+        const int wv = type == QMM_TYPE_Q8_0 ? 8 : 4;
+        FusedPlan split;
+        if (!gemv_fused_split_plan(type, w, 1, 1, wv, 1, &split) || !fq1_for(type, w, split)) break;
+        // (a plan forced by the tuning switches stays as forced)
+        if (fp.KS > 1 && (fp.W != wv || fp.spw != 1)) break;
+        m[n] = fq1_mat(a.src1, w, (float *)((uint8_t *)a.dst->buffer->ptr + a.dst->offs), wv, nullptr);
+        const size_t need = (size_t)gemv_fq1_tree_words(m[n]);
+        if (words + need > kTreeMinWords) break;
+        bool apart = !ranges_overlap(a.dst, a.src1);
+        const uint8_t * d0 = (const uint8_t *)m[n].dst, * d1 = d0 + (size_t)w.M * 4;
+        for (int i = 0; i <= n && apart; ++i) {
+            const Fq1Mat & o = m[i];
+            const size_t image = (size_t)((o.M + kTileRows - 1) / kTileRows) * (size_t)o.G * (size_t)tile_group_bytes(type);
+            apart = !(d0 < o.base + image && o.base < d1);          // (a dst over a weight image)
+            if (i == n) break;
+            const uint8_t * e0 = (const uint8_t *)o.dst, * e1 = e0 + (size_t)o.M * 4;
+            const uint8_t * mine = m[n].base, * mend = mine + (size_t)w.ntiles * (size_t)w.G * (size_t)w.tg;
+            apart = apart && !ranges_overlap(a.dst, nodes[i].dst) && !ranges_overlap(a.dst, nodes[i].src1) &&
+                    !ranges_overlap(nodes[i].dst, a.src1) && !(e0 < mend && mine < e1);
+        }
+        if (!apart) break;
+        m[n].tree = reinterpret_cast<uint32_t *>(words);            // (its offset, until the slots are there)
+        words += need;
+        *W = wv;
+    }
+    if (n < 2) return 0;
+    if (words) {
+        if (ctx->tree_words < words && (ctx->capturing || ensure_tree(ctx, words))) return 0;
+        for (int i = 0; i < n; ++i) m[i].tree = ctx->tree + reinterpret_cast<size_t>(m[i].tree);
+    }
+    return n;
+}
+
 int qmm_graph_compute(qmm_ctx * ctx, const qmm_node * nodes, int n_nodes) {
     if (!ctx || (!nodes && n_nodes)) return QMM_ERR_INVALID;
     ctx->graph_gen++;
     ctx->in_graph = true;
     int rc = QMM_OK;
-    for (int i = 0; i < n_nodes && rc == QMM_OK; ++i) {
+    for (int i = 0; i < n_nodes && rc == QMM_OK;) {
         const qmm_node & n = nodes[i];
-        if (n.op == QMM_OP_MUL_MAT) rc = qmm_mul_mat(ctx, n.src0, n.src1, n.dst);
-        else if (n.op == QMM_OP_MUL_MAT_ID) rc = qmm_mul_mat_id(ctx, n.src0, n.src1, n.ids, n.dst);
-        else rc = fail(ctx, QMM_ERR_UNSUPPORTED, "graph node %d: unsupported op %d", i, n.op);
-        // a node that writes over the cached activations' source invalidates them
-        if (ctx->key.valid) {
-            qmm_tensor src{};
-            src.type = QMM_TYPE_F32;
-            src.buffer = const_cast<qmm_buffer *>(ctx->key.buf);
-            src.offs = ctx->key.offs;
-            memcpy(src.ne, ctx->key.ne, sizeof(src.ne));
-            memcpy(src.nb, ctx->key.nb, sizeof(src.nb));
-            if (ranges_overlap(&src, n.dst)) ctx->key.valid = false;
+        int done = 1;
+        Fq1Mat m[kFq1Max];
+        int W = 0;
+        if (n.op == QMM_OP_MUL_MAT && n.src1 && n.src1->ne[1] == 1 && i + 1 < n_nodes &&
+            (done = fq1_run(ctx, nodes + i, n_nodes - i, m, &W)) > 1) {
+            rc = hipSetDevice(ctx->device) == hipSuccess ? fq1_launch(ctx, n.src0->type, m, done, W)
+                                                         : fail(ctx, QMM_ERR_DEVICE, "graph_compute: hipSetDevice");
+            ctx->path = "gemv-fq";
+        } else {
+            done = 1;
+            if (n.op == QMM_OP_MUL_MAT) rc = qmm_mul_mat(ctx, n.src0, n.src1, n.dst);
+            else if (n.op == QMM_OP_MUL_MAT_ID) rc = qmm_mul_mat_id(ctx, n.src0, n.src1, n.ids, n.dst);
+            else rc = fail(ctx, QMM_ERR_UNSUPPORTED, "graph node %d: unsupported op %d", i, n.op);
         }
-        if (ctx->rkey.valid && ranges_overlap(&ctx->rkey.ids, n.dst)) ctx->rkey.valid = false;
+        for (const int end = i + done; i < end; ++i) {
+            // a node that writes over the cached activations' source invalidates them
+            const qmm_tensor * dst = nodes[i].dst;
+            if (ctx->key.valid) {
+                qmm_tensor src{};
+                src.type = QMM_TYPE_F32;
+                src.buffer = const_cast<qmm_buffer *>(ctx->key.buf);
+                src.offs = ctx->key.offs;
+                memcpy(src.ne, ctx->key.ne, sizeof(src.ne));
+                memcpy(src.nb, ctx->key.nb, sizeof(src.nb));
+                if (ranges_overlap(&src, dst)) ctx->key.valid = false;
+            }
+            if (ctx->rkey.valid && ranges_overlap(&ctx->rkey.ids, dst)) ctx->rkey.valid = false;
+        }
     }
     ctx->in_graph = false;
     return rc;
