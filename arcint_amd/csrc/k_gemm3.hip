@@ -1,7 +1,7 @@
 // k_gemm3.hip - the streaming prefill GEMMs on gfx950 v_mfma_i32_32x32x32_i8: Q4_K
 // (k_gemm3_q4k, also the grouped MoE GEMM) and the block types with one float scale per 32
-// weights, Q4_0, Q8_0 and IQ4_NL (k_gemm3_blk), weights streamed by each wave; one product, or a
-// gate/up pair with its GLU in one launch (PAIR).
+// weights, Q4_0, Q8_0 and IQ4_NL (k_gemm3_blk; k_gemm3_wide where a launch is large), weights streamed
+// by each wave; one product, or a gate/up pair with its GLU in one launch (PAIR).
 //
 // Role of the reference's int8 prefill GEMMs (kernel_mul_mm_kq2d_q4_0_i8, P0099:377-455;
 // kernel_mul_mm_kq2d_q4_K_i8, P01:1919-2024) and its fp16 tile kernel for Q8_0
@@ -46,6 +46,7 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int kMagic = 0x4B400000;       // float 12582912: its bits + i are the float 12582912 + i, |i| < 2^22
 // Buffer loads: a wave-uniform resource (base and byte size in scalar registers), a 32-bit lane
@@ -93,15 +94,17 @@ __device__ __forceinline__ uint32_t bld4(__amdgpu_buffer_rsrc_t r, uint32_t voff
 //    next super-block's as soon as its two sub-blocks are done.
 constexpr int kKQStage = 18 * 1024;           // A [2 tiles][8 sub-blocks][1 KB], S [2][32][16], D [2][32] f32 (1 KB slot)
 constexpr int kKQMaxWaves = 12;
+constexpr int kWideU = 4;                     // waves of a 64 x 64 work-group
 // every wave stages ceil(18 / U) units of 1 KB per super-block, the same count on every wave and
 // every iteration (so the barrier waits for exactly these loads, not the weight loads issued
 // after them); units past 18 read nothing (out of range) into a 1 KB slot after the stages
 __host__ __device__ constexpr int kq_units(int U) { return (18 + U - 1) / U; }
-// s_waitcnt immediates (gfx9 encoding): vmcnt 5 / 8 / 9 (bits 3:0, 15:14), expcnt and lgkmcnt not
+// s_waitcnt immediates (gfx9 encoding): vmcnt 5 / 8 / 9 / 18 (bits 3:0, 15:14), expcnt and lgkmcnt not
 // waited on
 constexpr int kVmcnt5 = 5 | (0x7 << 4) | (0xF << 8);
 constexpr int kVmcnt8 = 8 | (0x7 << 4) | (0xF << 8);
 constexpr int kVmcnt9 = 9 | (0x7 << 4) | (0xF << 8);
+constexpr int kVmcnt18 = (18 & 15) | ((18 >> 4) << 14) | (0x7 << 4) | (0xF << 8);
 
 struct KQParams {
     WView w;
@@ -266,6 +269,17 @@ __device__ __forceinline__ KQWave kq_wave(const KQParams & p, uint32_t mb, int U
     return v;
 }
 
+// a column tile's 16 sums of row m to their columns (dense, non-temporal): those of live
+__device__ __forceinline__ void kq_store(const KQParams & p, uint32_t nb, int c, uint32_t i2, uint32_t i3, int64_t m, int h,
+                                         uint32_t live, const float (&val)[16]) {
+    float * dst = p.dst + (int64_t)i2 * p.bt.d_nb2 + (int64_t)i3 * p.bt.d_nb3 + m;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int64_t n = (2 * (int64_t)nb + c) * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+        if (n < p.N && ((live >> r) & 1u)) __builtin_nontemporal_store(val[r], dst + n * p.bt.d_nb1);
+    }
+}
+
 // The end of a block, a wave's 32 sums per lane (row m, the column pair's two tiles) complete over
 // its K slice:
 //  * K slices 1.. add theirs into slice 0's through LDS, in slice order;
@@ -363,12 +377,7 @@ __device__ __forceinline__ void kq_finish(const KQParams & p, uint8_t * lds, uin
             for (int r = 0; r < 16; ++r)
                 __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(val[r]), dres, (int)off[r], 0, 0);
         } else {
-            float * dst = p.dst + (int64_t)i2 * p.bt.d_nb2 + (int64_t)i3 * p.bt.d_nb3 + m;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int64_t n = (2 * (int64_t)nb + c) * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-                if (n < p.N && ((live >> r) & 1u)) __builtin_nontemporal_store(val[r], dst + n * p.bt.d_nb1);
-            }
+            kq_store(p, nb, c, i2, i3, m, h, live, val);
         }
     }
 }
@@ -1360,6 +1369,190 @@ __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_blk(KQParams p) {
               TYPE == QMM_TYPE_Q4_0 ? 0.0625f : 1.0f, out0, out1);
 }
 
+// ---- Q4_0, Q8_0, IQ4_NL, large launches: waves of 64 rows x 64 columns ----------------------
+// k_gemm3_blk's step on two row units a wave: both halves of an image tile, or (PAIR) one half of the
+// gate's tile and the same half of up's, so a pair's two sums meet in the lane's registers.  Bound by
+// the work each block-tile issues, which adds up at the chip's sustained power (per SIMD: an MFMA 18.5
+// ns, a VALU instruction 0.85, an LDS read of 16 bytes a lane 6.3): k_gemm3_blk's 37 VALU and 5 LDS
+// reads a block-tile are 84 ns, and 4 of the 5 reads bring the column scales.  Here one read of the
+// operand and of the scales serves both row units: 2.5 a block-tile.
+//  * 4 waves a work-group (one stage, one K slice), two work-groups a CU: two waves a SIMD with up to
+//    256 registers (64 sums, 32 MFMA results, 32 of weights: PF = 4 blocks ahead instead of 8).
+//  * Measured, op us, against k_gemm3_blk: Q4_0 11008 x 4096 x 2048 250 -> 239, 4096 x 11008 x 2048
+//    260 -> 237, its gate/up pair at 2048 of 11008 x 4096 with the down product 730 -> 676; Q8_0 16384 x
+//    4096 x 512 110 -> 89; IQ4_NL 4096 x 14336 x 2000 385 -> 350.  Where it leaves CUs without two
+//    work-groups it loses: Q4_0 11008 x 4096 x 512 (344 work-groups) 67 -> 78 (kq_wide_shape).
+template <int TYPE, bool PAIR>
+__global__ __launch_bounds__(64 * kWideU, 2) void k_gemm3_wide(KQParams p) {
+    constexpr bool Q8 = TYPE == QMM_TYPE_Q8_0;
+    constexpr bool NLQ = TYPE == QMM_TYPE_IQ4_NL;
+    constexpr int kDch = Q8 ? 16 : 8;                         // chunk plane of the block scales
+    constexpr int U = kWideU, PF = 4;                         // (weights PF blocks ahead)
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, j32 = lane & 31;
+    const int u = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+    uint32_t L;
+    int piece;
+    if (!kq_block(p, blockIdx.x, L, piece)) return;           // uniform over the work-group
+    const uint32_t mb = L / (uint32_t)p.nbn, nb = L - mb * (uint32_t)p.nbn;
+    const uint32_t bz = blockIdx.y;
+    const uint32_t i2 = bz % (uint32_t)p.bt.ne12, i3 = bz / (uint32_t)p.bt.ne12;
+    const int64_t mat = (int64_t)(i2 / (uint32_t)p.bt.r2) + (int64_t)(i3 / (uint32_t)p.bt.r3) * p.bt.ne02;
+    // the wave's rows: an image tile's two halves, or one half of the gate's tile and of up's
+    const int64_t raw = (int64_t)mb * U + u, units = PAIR ? 2 * p.w.ntiles : p.w.ntiles;
+    const bool row_ok = raw < units;                          // (a missing unit computes a copy, stores nothing)
+    const int64_t unit_ = row_ok ? raw : units - 1;
+    const int64_t mtile = PAIR ? unit_ >> 1 : unit_;
+    const int t = PAIR ? (int)(unit_ & 1) : 0;
+    const int64_t ct0 = (int64_t)bz * p.ntb + 2 * (int64_t)nb; // the pair's first column tile
+    const int64_t nct = std::min<int64_t>(2, p.ntb - 2 * (int64_t)nb);
+    const int ng = (int)p.nsb;                                // groups (256 weights) along K
+    const int64_t nblk = 8 * p.nsb;                           // blocks per activation column
+
+    WView wu = p.w;
+    if (PAIR) wu.base = p.up;
+    const uint32_t wbytes = (uint32_t)(p.w.G * p.w.tg);
+    const __amdgpu_buffer_rsrc_t wbuf0 = buffer_rsrc(tile_group(p.w, mat, mtile, 0), wbytes);
+    const __amdgpu_buffer_rsrc_t wbuf1 = PAIR ? buffer_rsrc(tile_group(wu, mat, mtile, 0), wbytes) : wbuf0;
+    const __amdgpu_buffer_rsrc_t abuf = buffer_rsrc(p.tA + ct0 * nblk * 1024, (uint32_t)(nct * nblk * 1024));
+    const __amdgpu_buffer_rsrc_t dbuf = buffer_rsrc(p.tD + ct0 * nblk * 32, (uint32_t)(nct * nblk * 128));
+    const uint32_t lane16 = (uint32_t)lane * 16;
+
+    constexpr int NU = kq_units(U);
+    constexpr uint32_t kOut = 0x7ff00000u;
+    const uint32_t a_stride = (uint32_t)(nblk * 1024), d_stride = (uint32_t)(nblk * 128);
+    const uint32_t lane16b = lane16 + a_stride;               // (the second column tile)
+    // (picked once, as scalars: a stage is NU loads on a straight line.  Behind a branch per kind of
+    // unit the compiler counts none of them as issued, and its waits for the weights drain them too)
+    const uint32_t d_lane = u < 2 ? lane16 + (uint32_t)u * d_stride : kOut;
+    const uint32_t d_lds = u < 2 ? (uint32_t)(16 + u) * 1024 : 2 * kKQStage, d_buf = u < 2 ? (uint32_t)kKQStage : 0;
+    auto stage = [&](int s, int b) {
+#pragma unroll
+        for (int i = 0; i < NU - 1; ++i) {
+            const int unit = u + i * U;                       // wave-uniform, below 16
+            dma16(abuf, lds + b * kKQStage + unit * 1024, unit >> 3 ? lane16b : lane16,
+                  (uint32_t)s * 8192 + (uint32_t)(unit & 7) * 1024);
+        }
+        dma16(dbuf, lds + d_lds + (uint32_t)b * d_buf, d_lane, (uint32_t)s * 1024);
+    };
+
+    const uint32_t tgs = (uint32_t)p.w.tg;
+    const uint32_t row16 = (uint32_t)(32 * t + j32) * 16;
+    auto wplane = [&](int jb) -> uint32_t { return (uint32_t)(Q8 ? 2 * jb + h : jb) * kChunk; };
+    auto wld = [&](int i, uint32_t plane, uint32_t soff) {
+        return i ? bld16(wbuf1, row16 + (PAIR ? 0u : 512u) + plane, soff) : bld16(wbuf0, row16 + plane, soff);
+    };
+    uint4 wq[2][PF], wd[2];
+    v16f out[2][2] = {};                                      // [row unit][column tile]
+    v16i magic;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) magic[r] = kMagic;
+    const uint32_t nshift = (uint32_t)(4 - 4 * h);            // Q4_0: the lane half's nibble to the high nibble
+    const Iq4Regs kr = iq4_regs();                             // IQ4_NL: the codebook in VGPRs
+    auto unpack = [&](const uint4 & x) -> v4i {
+        if constexpr (Q8) return v4i{ (int)x.x, (int)x.y, (int)x.z, (int)x.w };
+        else if constexpr (NLQ) {
+            const uint32_t sh = 4u * (uint32_t)h;
+            return v4i{ (int)iq4_lookup_r(x.x >> sh, kr), (int)iq4_lookup_r(x.y >> sh, kr),
+                        (int)iq4_lookup_r(x.z >> sh, kr), (int)iq4_lookup_r(x.w >> sh, kr) };
+        } else {
+            return v4i{ (int)(((x.x << nshift) & 0xF0F0F0F0u) ^ 0x80808080u),
+                        (int)(((x.y << nshift) & 0xF0F0F0F0u) ^ 0x80808080u),
+                        (int)(((x.z << nshift) & 0xF0F0F0F0u) ^ 0x80808080u),
+                        (int)(((x.w << nshift) & 0xF0F0F0F0u) ^ 0x80808080u) };
+        }
+    };
+    auto consume = [&](v16f & acc, const v16i & e, float dw, float nm, const float (&dx)[16]) {
+        v16f tv;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int iv = e[r];
+            tv[r] = __builtin_fmaf(__builtin_bit_cast(float, iv), dw, nm);
+        }
+        asm volatile("" : "+v"(tv));
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] = __builtin_fmaf(tv[r], dx[r], acc[r]);
+    };
+    auto compute = [&](int b, int s) {
+        const uint8_t * S = lds + b * kKQStage;
+        const uint4 dd[2] = { wd[0], wd[1] };
+        const uint32_t sc = (uint32_t)s * tgs, sn = (uint32_t)std::min(s + 1, ng - 1) * tgs;   // the next group (clamped)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) wd[i] = wld(i, kDch * kChunk, sn);
+#pragma unroll
+        for (int jb = 0; jb < 8; ++jb) {
+            v4i bop[2];
+            float dw[2], nm[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                bop[i] = unpack(wq[i][jb % PF]);
+                const uint32_t dword = jb < 2 ? dd[i].x : jb < 4 ? dd[i].y : jb < 6 ? dd[i].z : dd[i].w;
+                dw[i] = h2f((dword >> (16 * (jb & 1))) & 0xffffu);
+                asm volatile("" : "+v"(dw[i]));               // f32 operands (no fp16 source folding)
+                nm[i] = -12582912.0f * dw[i];
+                wq[i][jb % PF] = wld(i, wplane((jb + PF) % 8), jb + PF < 8 ? sc : sn);
+            }
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const v4i a = *reinterpret_cast<const v4i *>(S + c * 8192 + jb * 1024 + lane16);
+                const v16i e0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, bop[0], magic, 0, 0, 0);
+                const v16i e1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, bop[1], magic, 0, 0, 0);
+                float dx[16];
+#pragma unroll
+                for (int q4 = 0; q4 < 4; ++q4) {
+                    const v4f v = *reinterpret_cast<const v4f *>(S + 16384 + c * 1024 + jb * 128 + h * 64 + 16 * q4);
+                    dx[4 * q4] = v.x;
+                    dx[4 * q4 + 1] = v.y;
+                    dx[4 * q4 + 2] = v.z;
+                    dx[4 * q4 + 3] = v.w;
+                }
+                consume(out[0][c], e0, dw[0], nm[0], dx);
+                consume(out[1][c], e1, dw[1], nm[1], dx);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    stage(0, 0);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) wd[i] = wld(i, kDch * kChunk, 0);   // (in the steps' order: their waits count on it)
+#pragma unroll
+    for (int jb = 0; jb < PF; ++jb)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) wq[i][jb] = wld(i, wplane(jb), 0);
+    __syncthreads();
+    for (int s = 0; s < ng; ++s) {                            // uniform over the work-group
+        stage(std::min(s + 1, ng - 1), (s + 1) & 1);          // (past the end: a copy nobody reads)
+        __builtin_amdgcn_sched_barrier(0);                    // the LDS loads go out before the weight loads
+        compute(s & 1, s);
+        // this wave's LDS loads are complete once at most the 18 weight loads issued after them
+        // are outstanding; the barrier then publishes them to the other waves
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(kVmcnt18);
+        __syncthreads();
+    }
+
+    if (!row_ok) return;
+    constexpr float scale = TYPE == QMM_TYPE_Q4_0 ? 0.0625f : 1.0f;   // (Q4_0 codes carried 16 (q - 8))
+#pragma unroll
+    for (int i = PAIR ? 1 : 0; i < 2; ++i) {
+        const int64_t m = mtile * kTileRows + 32 * (PAIR ? t : i) + j32;
+        if (m >= p.w.M) continue;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            float gv[16], val[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                val[r] = out[i][c][r] * scale;
+                gv[r] = out[0][c][r] * scale;
+            }
+            if constexpr (PAIR) glu_switch(p.glu, gv, val);
+            kq_store(p, nb, c, i2, i3, m, h, 0xffffu, val);
+        }
+    }
+}
+
 // one launch of kernel K
 template <typename F>
 hipError_t launch_k(F * k, const KQParams & q, const G3Shape & sh, const dim3 & g, const dim3 & b, hipStream_t s,
@@ -1399,6 +1592,12 @@ hipError_t launch_u(const KQParams & q, const G3Shape & sh, const dim3 & g, cons
 template <int TYPE, bool GATHER>
 hipError_t launch_t(const KQParams & q, const G3Shape & sh, const dim3 & g, const dim3 & b, hipStream_t s,
                     const KTime * kt) {
+    if constexpr (!GATHER && (TYPE == QMM_TYPE_Q4_0 || TYPE == QMM_TYPE_Q8_0 || TYPE == QMM_TYPE_IQ4_NL)) {
+        if (sh.R == 64) {
+            if (q.up) return launch_k(&k_gemm3_wide<TYPE, true>, q, sh, g, b, s, kt);
+            return launch_k(&k_gemm3_wide<TYPE, false>, q, sh, g, b, s, kt);
+        }
+    }
     return q.up ? launch_u<TYPE, GATHER, true>(q, sh, g, b, s, kt) : launch_u<TYPE, GATHER, false>(q, sh, g, b, s, kt);
 }
 
@@ -1589,6 +1788,47 @@ bool kq_pair_shape(const WView & w, int64_t N, int64_t nbatch, G3Shape * sh, boo
     if (us) *us = best;
     return best >= 0 && sh->mbn * ncp < 0x7fffffff && sh->lds <= 160 * 1024 && sh->threads <= 64 * kKQMaxWaves;
 }
+// Launch shape of the 64 x 64 waves (k_gemm3_wide), and whether it is taken: when its estimated time is
+// below that of 32-row waves, us (their own estimate for a gate/up pair, else by their count).  In us a
+// step of 256 weights: two work-groups a CU take w a step; 12 waves of 32 rows a CU take n.  Rounds
+// of 512 work-groups: up to 256 left over run one a CU, in about half a round (a lone work-group has
+// the CU to itself), more of them nearly a whole one.  Measured (8192 x 4096, wide / narrow us): Q4_0
+// 1024 columns (1 round) 87 / 101, 1088 (1.06) 131 / 106, 1408 (1.38) 133 / 128, 1536 (1.5) 134 / 139,
+// 1664 (1.63) 157 / 153, 2048 (2) 167 / 186; Q8_0 1024 87 / 114, 1280 (1.25) 131 / 131, 1536 134 / 155;
+// IQ4_NL 768 (0.75) 90 / 85, 1024 100 / 115; FFN blocks by pairs: Q4_0 256 columns (0.5) 101 / 96, 448 137 /
+// 157, 576 (1.13) 200 / 189, 768 (1.5) 228 / 235, Q8_0 256 100 / 111, 512 150 / 187.
+bool kq_wide_shape(int type, const WView & w, int64_t N, int64_t nbatch, G3Shape * sh, bool pair, double us) {
+    const int64_t ncp = ((N + 31) / 32 + 1) / 2, units = pair ? 2 * w.ntiles : w.ntiles;
+    const int64_t mbn = (units + kWideU - 1) / kWideU, nwg = mbn * ncp;
+    const int env = env_int3("QMM_GEMM3_WIDE", -1);           // 0 never, 1 always
+    if (env == 0 || (env < 0 && env_int3(pair ? "QMM_GEMM3_PAIR" : "QMM_GEMM3_KQ", -1) >= 0)) return false;
+    if (env < 0) {
+        const bool q4 = type == QMM_TYPE_Q4_0, q8 = type == QMM_TYPE_Q8_0;
+        const double wstep = q4 ? 5.2 : q8 ? 5.1 : 5.75, nstep = q4 ? 4.36 : q8 ? 5.0 : 4.95;
+        const int64_t whole = nwg * nbatch / 512, rest = nwg * nbatch % 512;
+        const double rounds = (double)whole + (rest == 0 ? 0 : whole == 0 ? (rest <= 256 ? 0.66 : 1.0) : rest <= 256 ? 0.55 : 0.9);
+        // (a pair's own estimate is at Q4_0's 4.25 a step)
+        const double narrow = pair ? us * (q4 ? 1.0 : nstep / 4.25)
+                                   : (double)(2 * w.ntiles * ncp * nbatch) / 3072 * nstep * (double)w.G;
+        if (rounds * wstep * (double)w.G > 0.975 * narrow) return false;
+    }
+    *sh = G3Shape{};
+    sh->C = 2;
+    sh->R = 64;
+    sh->SB = 8;
+    sh->U = kWideU;
+    sh->KS = 1;
+    sh->sps = sh->nst = sh->pk = (int)w.G;
+    sh->mbn = mbn;
+    sh->nbn = ncp;
+    sh->threads = 64 * kWideU;
+    sh->lds = 2 * kKQStage + 1024;
+    sh->ts = 1;
+    sh->full = nwg;
+    sh->fchunk = (nwg + 7) / 8;
+    sh->workgroups = 8 * sh->fchunk * nbatch;
+    return nwg < 0x7fffffff;
+}
 }  // namespace
 
 bool gemm3_id_supported(int type) {
@@ -1653,7 +1893,13 @@ bool gemm3_shape(int type, const WView & w, int64_t N, int64_t nbatch, G3Shape *
     if (!gemm3_supported(type) || N <= 0 || nbatch <= 0 || nbatch > 65535 || w.G <= 0 || w.ntiles <= 0) return false;
     // (the K-quant frame's launch rule for the super-block types; the block types' for the rest)
     const bool kframe = type == QMM_TYPE_Q4_K || type == QMM_TYPE_Q6_K || type == QMM_TYPE_Q5_K || type == QMM_TYPE_IQ4_XS;
-    return pair ? kq_pair_shape(w, N, nbatch, sh, !kframe, us) : kq_shape(w, N, nbatch, sh, !kframe);
+    G3Shape wide;
+    double est = 0;
+    if (pair && !kq_pair_shape(w, N, nbatch, sh, !kframe, &est)) return false;
+    if (us) *us = est;
+    if (!pair && !kq_shape(w, N, nbatch, sh, !kframe)) return false;
+    if (!kframe && kq_wide_shape(type, w, N, nbatch, &wide, pair, est)) *sh = wide;
+    return true;
 }
 
 size_t gemm3_tree_words(const G3Shape & sh) {
