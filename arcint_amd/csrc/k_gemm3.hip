@@ -1627,14 +1627,15 @@ namespace {
 // form, kKQOneSlice); only = -2: every candidate but that one (the grouped mode's split form:
 // there it tied with (2, 2, 3) on 128 experts x 32 pairs and measured 54.8 against 46.8 us)
 constexpr int kKQOneSlice = 4;                                // (4, 1, 3) in the candidates below
+constexpr int kKQCands = 6;
 bool kq_shape_ncp(const WView & w, int64_t ncp, int64_t nbatch, G3Shape * sh, bool blk, bool tail, int only, bool pair) {
     struct Cand { int U, KS, per_cu; };
-    static const Cand cands[] = { { 12, 1, 1 }, { 6, 2, 1 }, { 4, 3, 1 }, { 3, 4, 1 }, { 4, 1, 3 }, { 2, 2, 3 } };
+    static const Cand cands[kKQCands] = { { 12, 1, 1 }, { 6, 2, 1 }, { 4, 3, 1 }, { 3, 4, 1 }, { 4, 1, 3 }, { 2, 2, 3 } };
     const int64_t nrh = 2 * w.ntiles, G = w.G;
     const int cus = 256;
     int64_t best = -1;
     const int forced = env_int3("QMM_GEMM3_KQ", -1);           // index into cands (tuning)
-    for (int i = 0; i < (int)(sizeof(cands) / sizeof(cands[0])); ++i) {
+    for (int i = 0; i < kKQCands; ++i) {
         if (forced >= 0 && i != forced) continue;
         if (forced < 0 && only >= 0 && i != only) continue;
         if (forced < 0 && only == -2 && i == kKQOneSlice) continue;
@@ -1709,8 +1710,48 @@ bool kq_shape_ncp(const WView & w, int64_t ncp, int64_t nbatch, G3Shape * sh, bo
     sh->workgroups = 8 * (sh->fchunk + sh->tchunk) * nbatch;
     return sh->mbn * ncp < 0x7fffffff && sh->lds <= 160 * 1024 && sh->threads <= 64 * kKQMaxWaves;
 }
-bool kq_shape(const WView & w, int64_t N, int64_t nbatch, G3Shape * sh, bool blk) {
-    return kq_shape_ncp(w, ((N + 31) / 32 + 1) / 2, nbatch, sh, blk, true, -1, false);
+
+// Op time in us of one product in shape sh (from kq_shape_ncp, a launch below one round of 4-wave
+// blocks), the activation pre-pass and the launches in it: steps along K of the busiest CU times a
+// step's time.  A step of a wave's 32 rows x 64 columns takes c us where three waves share a SIMD 3.26
+// ways (t, as in kq_pair_shape); a piece reads and writes its 8 KB of sums a wave through memory.
+double kq_small_us(int type, const G3Shape & sh, int64_t ncp) {
+    const double c = type == QMM_TYPE_Q4_K ? 1.06 : type == QMM_TYPE_Q6_K ? 1.12 : type == QMM_TYPE_Q5_K ? 1.25
+                   : type == QMM_TYPE_IQ4_XS ? 1.35 : type == QMM_TYPE_Q8_0 ? 1.5 : 1.4;
+    auto t = [](double waves) { return waves <= 1 ? 2.0 : waves <= 2 ? 1.6 + 0.4 * waves : 0.68 + 0.86 * waves; };
+    const int64_t nwg = sh.mbn * ncp, cus = 256;
+    const int waves = sh.U * sh.KS;
+    const double load = (double)((nwg * sh.ts + cus - 1) / cus);  // blocks or pieces on the busiest CU
+    const double at = std::min(load, waves <= 4 ? 3.0 : 1.0);     // ... at a time
+    const double run = c * sh.sps * t(at * waves / 4) * (load / at);
+    if (sh.ts == 1) return 8.5 + run + 0.6 * (sh.KS - 1);
+    return 13.0 + 0.92 * run / sh.sps * sh.pk + 0.0055 * (double)(nwg * sh.ts * sh.U);
+}
+
+// Launch shape of one product.  Below one round of 4-wave blocks (256 of them, one batch) the rounds
+// that kq_shape_ncp counts do not tell the candidates apart: one wave a SIMD takes 2 c a step, three
+// 3.3 c, and blocks in pieces along K fill CUs that whole ones leave idle.  There the smallest estimate
+// wins, and *us is it (else -1), for K from 8192 on.  Measured (op us, KS = 4 as the rounds chose /
+// 4-wave blocks in pieces along K): Q5_K 5120 x 17408 at 40 columns 79 / 54, at 128 81 / 68; IQ4_XS 4096 x
+// 14336 at 128 71 / 53, Q8_0 67 / 58, Q4_0 4096 x 11008 at 128 51 / 45; but Q4_K 5120 x 17408 at 256 74 /
+// 81.  A shorter K's pieces have too few steps for what they exchange, and the rounds' choice is the
+// best or within 4 % (Q4_K 5120 x 6144 at 128 31 / 34, 4096 x 4096 24 / 28, Q8_0 5761 x 2880 at 203 25 /
+// 49).  whole: no tree slots for pieces, the rounds decide.
+bool kq_shape(int type, const WView & w, int64_t N, int64_t nbatch, G3Shape * sh, bool blk, bool whole, double * us) {
+    const int64_t ncp = ((N + 31) / 32 + 1) / 2;
+    *us = -1;
+    if (whole || nbatch != 1 || w.G < 32 || (2 * w.ntiles + 3) / 4 * ncp >= 256 || env_int3("QMM_GEMM3_KQ", -1) >= 0 ||
+        env_int3("QMM_GEMM3_TAIL", 1) != 1)
+        return kq_shape_ncp(w, ncp, nbatch, sh, blk, true, -1, false);
+    for (int i = 0; i < kKQCands; ++i) {
+        G3Shape c{};
+        if (!kq_shape_ncp(w, ncp, nbatch, &c, blk, true, i, false)) continue;
+        const double v = kq_small_us(type, c, ncp);
+        if (*us >= 0 && v >= *us) continue;
+        *us = v;
+        *sh = c;
+    }
+    return *us >= 0;
 }
 
 // Launch shape of a dense gate/up pair and its estimated time in us (kernel only), the smallest of
@@ -1889,15 +1930,15 @@ hipError_t launch_gemm3_id(int type, const WView & w, const ActBuf & a, const Ge
 }
 
 // Launch shape of both kernels (kq_shape): U row-half waves per K slice x KS slices.
-bool gemm3_shape(int type, const WView & w, int64_t N, int64_t nbatch, G3Shape * sh, bool pair, double * us) {
+bool gemm3_shape(int type, const WView & w, int64_t N, int64_t nbatch, G3Shape * sh, bool pair, double * us, bool whole) {
     if (!gemm3_supported(type) || N <= 0 || nbatch <= 0 || nbatch > 65535 || w.G <= 0 || w.ntiles <= 0) return false;
     // (the K-quant frame's launch rule for the super-block types; the block types' for the rest)
     const bool kframe = type == QMM_TYPE_Q4_K || type == QMM_TYPE_Q6_K || type == QMM_TYPE_Q5_K || type == QMM_TYPE_IQ4_XS;
     G3Shape wide;
     double est = 0;
     if (pair && !kq_pair_shape(w, N, nbatch, sh, !kframe, &est)) return false;
+    if (!pair && !kq_shape(type, w, N, nbatch, sh, !kframe, whole, &est)) return false;
     if (us) *us = est;
-    if (!pair && !kq_shape(w, N, nbatch, sh, !kframe)) return false;
     if (!kframe && kq_wide_shape(type, w, N, nbatch, &wide, pair, est)) *sh = wide;
     return true;
 }
@@ -1907,9 +1948,9 @@ size_t gemm3_tree_words(const G3Shape & sh) {
 }
 
 hipError_t launch_gemm3(int type, const WView & w, const TiledAct & a, int64_t nbatch, const GemmBatch & bt,
-                        float * dst, hipStream_t s, const KTime * kt, uint32_t * tree, const uint8_t * up, int glu) {
+                        float * dst, hipStream_t s, const KTime * kt, uint32_t * tree, const uint8_t * up, int glu, bool whole) {
     G3Shape sh;
-    if ((glu >= 0) != (up != nullptr) || !gemm3_shape(type, w, a.N, nbatch, &sh, up != nullptr) || !a.A || !a.D || a.nblk != w.G * 8 || a.ntb != (a.N + 31) / 32 ||
+    if ((glu >= 0) != (up != nullptr) || !gemm3_shape(type, w, a.N, nbatch, &sh, up != nullptr, nullptr, whole) || !a.A || !a.D || a.nblk != w.G * 8 || a.ntb != (a.N + 31) / 32 ||
         a.ntiles != a.ntb * nbatch || a.vdt != vec_dot_type(type))
         return hipErrorInvalidValue;
     if ((type == QMM_TYPE_Q4_K || type == QMM_TYPE_Q5_K) && !a.S) return hipErrorInvalidValue;

@@ -312,6 +312,12 @@ int gemm3_tree(qmm_ctx * ctx, const G3Shape & g3, uint32_t ** tree) {
     return QMM_OK;
 }
 
+// whether a product's tail pieces would have no slots: a capture that would have to grow them
+bool gemm_whole(const qmm_ctx * ctx, int type, const WView & w, int64_t N, int64_t nbatch) {
+    G3Shape g3;
+    return ctx->capturing && gemm3_shape(type, w, N, nbatch, &g3) && ctx->tree_words < gemm3_tree_words(g3);
+}
+
 F32Cols f32_cols(const qmm_tensor * t) {
     F32Cols c;
     c.base = (const char *)t->buffer->ptr + t->offs;
@@ -892,27 +898,47 @@ static int64_t gemm_min_cols(int type) {
     return gemv_mma_supported(type) ? kMmaMaxCols + 1 : 16;
 }
 
-// MUL_MAT on the GEMM: from gemm_min_cols, when the streaming GEMM's launch gives every SIMD a
-// wave (rows x column units x K slices >= 1024); with fewer (down to 512) when the GEMV would
-// stream enough weight bytes over its passes (32 columns a pass on the MFMA GEMV, 8 on v_dot4):
-// 90 MB.  Q6_K, whose GEMM costs more per MAC, needs 400 MB at any wave count below 256 columns.
-// Else the GEMV's tasks, which split K over work-groups.  Measured (op us, GEMV / GEMM): Q4_K 17408 x 5120 at N = 40-64 44.7-50.8 / 31,
-// 12288 x 5120 at 48 30.0 / 30.0, 5120 x 6144 at 48-64 22-24 / 32-33; Q6_K 5120 x 17408 at 128
-// 96 / 116, at 192 141 / 122, the 151936-row head at 64 446 / 272; IQ4_XS 4096 x 14336 at 48-64
-// 35-38 / 73; Q5_K 17408 x 5120 at 16-48 62-135 / 34-36; config 3's shared expert (Q4_K 512 x
-// 2048, N = 256) 30.4 / 42.8.  QMM_GEMM_MIN_COLS, when set, decides alone.
-static bool use_gemm_for(int type, const WView & w, int64_t N, int64_t nbatch) {
+// Estimated op time in us of the GEMV's weight passes (32 columns each on the MFMA GEMV, 8 on v_dot4),
+// the activation pre-pass in it: a fixed part a pass, the image's bytes at a rate of the type's unpacking
+// work, a little by the columns.  Estimate / measured: Q4_K 5120 x 17408 at 40 columns 37 / 33,
+// at 77 53 / 53; IQ4_XS 4096 x 14336 at 77 45 / 41; Q8_0 4096 x 14336 at 77 44 / 40, at 128 58 / 65.
+static double gemv_passes_us(int type, const WView & w, int64_t N) {
+    const double mb = (double)(w.ntiles * w.G) * (double)w.tg / 1e6;
+    if (!gemv_mma_supported(type)) return 5.0 + (double)((N + 7) / 8) * (1.3 + mb / 2.7);
+    const double passes = (double)((N + kMmaMaxCols - 1) / kMmaMaxCols), cols = (double)N / passes;
+    const bool q8 = type == QMM_TYPE_Q8_0;
+    const double rate = q8 ? 8.0 : type == QMM_TYPE_Q4_K || type == QMM_TYPE_Q6_K ? 3.5 : type == QMM_TYPE_Q4_0 ? 2.8 : 2.7;
+    const double pass = (q8 ? 5.0 : 1.2) + mb / rate * (0.8 + 0.2 * cols / 26);
+    return 5.0 + passes * (std::max(pass, mb / 4.5) + 0.03 * cols);
+}
+
+// MUL_MAT on the GEMM, from gemm_min_cols.  When the streaming GEMM's launch gives every SIMD a
+// wave (rows x column units x K slices >= 1024); with fewer (down to 512) when the GEMV would stream
+// enough weight bytes over its passes (32 columns a pass on the MFMA GEMV, 8 on v_dot4): 90 MB.  Q6_K,
+// whose GEMM costs more per MAC, needs 400 MB at any wave count below 256 columns.  Else the GEMV's
+// tasks, which split K over work-groups.  Where the GEMM's shape was chosen by its time (K from 8192
+// on, below one round of its 4-wave blocks), that time has to be below 1.15 of the GEMV's as well (the
+// estimates' error; the waves are those of the shape that the rounds choose): Q8_0 4096 x 14336 at 40 columns 29 / 55, at 128 65 / 58; Q4_K 5120 x 17408 at 64 39 /
+// 47, at 128 70 / 59, 5570 x 8192 at 94 47 / 39; Q8_0 11861 x 14304 at 36 84 / 69.  For Q5_K it decides
+// alone (722 x 8704 at 308 95 / 41).  Measured (op us, GEMV / GEMM): Q4_K 17408 x 5120 at N =
+// 40-64 44.7-50.8 / 31, 12288 x 5120 at 48 30.0 / 30.0, 5120 x 6144 at 48-64 22-24 / 32-33; the Q6_K
+// 151936-row head at 64 446 / 272; Q5_K 17408 x 5120 at 16-48 62-135 / 34-36; config 3's shared expert
+// (Q4_K 512 x 2048, N = 256) 30.4 / 42.8.  QMM_GEMM_MIN_COLS, when set, decides alone.
+static bool use_gemm_for(int type, const WView & w, int64_t N, int64_t nbatch, bool whole = false) {
     if (N < gemm_min_cols(type)) return false;
     if (getenv("QMM_GEMM_MIN_COLS")) return true;
     G3Shape sh;
-    if (!gemm3_shape(type, w, N, nbatch, &sh)) return true;      // (the shared-tile GEMM)
+    double us = -1;
+    if (!gemm3_shape(type, w, N, nbatch, &sh, false, &us, whole)) return true;      // (the shared-tile GEMM)
+    if (us >= 0) gemm3_shape(type, w, N, nbatch, &sh, false, nullptr, true);        // (the rounds' launch)
     const int64_t waves = sh.mbn * sh.nbn * nbatch * sh.U * sh.KS;
     const int64_t per = gemv_mma_supported(type) ? kMmaMaxCols : 8;
     const double passes = (double)((N + per - 1) / per);
     const double bytes = (double)(w.ntiles * w.G) * (double)w.tg * (double)nbatch;
     if (type == QMM_TYPE_Q6_K && N < 256) return waves >= 512 && passes >= 2 && passes * bytes >= 400e6;
-    if (waves >= 1024) return true;
-    return waves >= 512 && passes >= 2 && passes * bytes >= 90e6;
+    const bool filled = waves >= 1024 || (waves >= 512 && passes >= 2 && passes * bytes >= 90e6);
+    if (us >= 0 && (filled || !gemv_mma_supported(type))) return us < 1.15 * gemv_passes_us(type, w, N);
+    return filled;
 }
 
 // A gate/up pair on the GEMM (one launch of both products): past one pass of the GEMV, when its
@@ -1185,7 +1211,8 @@ static bool try_fused_id(qmm_ctx * ctx, const qmm_tensor * src0, const qmm_tenso
 static int mul_mat_launch(qmm_ctx * ctx, const qmm_tensor * src0, const qmm_tensor * src1, const qmm_tensor * dst,
                           const WView & w, const FixedAct * fixed) {
     const int64_t N = src1->ne[1];
-    const bool use_gemm = use_gemm_for(src0->type, w, N, src1->ne[2] * src1->ne[3]);
+    const bool whole = fixed || gemm_whole(ctx, src0->type, w, N, src1->ne[2] * src1->ne[3]);
+    const bool use_gemm = use_gemm_for(src0->type, w, N, src1->ne[2] * src1->ne[3], whole);
     ActBuf a{};
     int rc;
     float * d = (float *)((uint8_t *)dst->buffer->ptr + dst->offs);
@@ -1204,7 +1231,7 @@ static int mul_mat_launch(qmm_ctx * ctx, const qmm_tensor * src0, const qmm_tens
     G3Shape g3;
     // weights streamed per wave, dst written once (the shape check is qmm_describe_mul_mat's, so
     // a shape the streaming kernel declines runs on the shared-tile GEMM below, as described)
-    if (use_gemm && gemm3_shape(src0->type, w, N, dn.ne12 * dn.ne13, &g3)) {
+    if (use_gemm && gemm3_shape(src0->type, w, N, dn.ne12 * dn.ne13, &g3, false, nullptr, whole)) {
         const int64_t nbatch = dn.ne12 * dn.ne13;
         TiledAct ta;
         if ((rc = quantize_src1_tiled(ctx, src0->type, src1, w.G, &ta, fixed))) return rc;
@@ -1222,7 +1249,7 @@ static int mul_mat_launch(qmm_ctx * ctx, const qmm_tensor * src0, const qmm_tens
         uint32_t * tree = nullptr;
         if (!fixed && (rc = gemm3_tree(ctx, g3, &tree))) return rc;
         if (!fixed && (rc = ktime_pair(ctx, &kt, &ktp))) return rc;
-        QMM_HIP(ctx, launch_gemm3(src0->type, w, ta, nbatch, bt, d, ctx->stream, ktp, tree));
+        QMM_HIP(ctx, launch_gemm3(src0->type, w, ta, nbatch, bt, d, ctx->stream, ktp, tree, nullptr, -1, whole));
         return ktime_done(ctx);
     }
     if (use_gemm) {

@@ -416,9 +416,11 @@ struct G3Shape {
     int ts, pk, tslots;
     int64_t fchunk, tchunk;        // per XCD: whole blocks, tail pieces
 };
-// pair: a gate/up pair in one launch (see launch_gemm3), us its estimated kernel time
+// pair: a gate/up pair in one launch (see launch_gemm3), us its estimated kernel time; one product: us
+// the op's estimated time where the shape was chosen by it, else -1; whole: tail pieces have no tree
+// slots to meet in, so the shape is not chosen for them (the same value at every call of one op)
 bool gemm3_shape(int type, const WView & w, int64_t N, int64_t nbatch, G3Shape * sh, bool pair = false,
-                 double * us = nullptr);
+                 double * us = nullptr, bool whole = false);
 // tree words the tail pieces of that launch meet in (0: no pieces)
 size_t gemm3_tree_words(const G3Shape & sh);
 // Grouped MoE GEMM (MUL_MAT_ID with many pairs per expert): the route's 64-column units
@@ -438,7 +440,7 @@ hipError_t launch_gemm3_id(int type, const WView & w, const ActBuf & a, const Ge
 // image and up the up matrix's (same shape and type): dst = act(gate) * up
 hipError_t launch_gemm3(int type, const WView & w, const TiledAct & a, int64_t nbatch, const GemmBatch & bt,
                         float * dst, hipStream_t s, const KTime * kt = nullptr, uint32_t * tree = nullptr,
-                        const uint8_t * up = nullptr, int glu = -1);
+                        const uint8_t * up = nullptr, int glu = -1, bool whole = false);
 
 // K slices the GEMM splits this product into; above 1 the slices add their
 // partial sums to dst with atomics, so dst must be zeroed first.
