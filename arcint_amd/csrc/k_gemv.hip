@@ -1652,12 +1652,12 @@ __global__ __launch_bounds__(1024) void k_gemv_fq(FqParams p) {
 }
 
 // ---- one-column dense products, one launch for up to kFq1Max of them --------------------------
-// k_gemv_fq's split form (one group a wave, W waves a work-group, KS work-groups per tile met in the
-// exchange tree) with nothing else in the kernel, for a list of independent products: work-group
+// k_gemv_fq's plans of one group a wave (W waves a work-group, KS work-groups per tile met in the
+// exchange tree, or K whole in one) with nothing else in the kernel, for a list of independent products: work-group
 // (x, y) is tile x - start[i] of product i, K slice y.  A decode step's projections are a few tens of MB
 // in all, and each launch ramps up and drains for ~4 us, which the next one waits for: Q5_K 12288, 1024
-// and 1024 x 5120 and 5120 x 6144 one after the other 29.2 us (26.8 on this kernel), in one launch 15.1.  Sums meet in the
-// same order as k_gemv_fq's (the same bits).
+// and 1024 x 5120 and 5120 x 6144 one after the other 29.2 us (26.8 on this kernel), in one launch 15.1.  Each product
+// keeps the W its own plan has, so its sums meet in the same order as k_gemv_fq's (the same bits).
 struct Fq1Params {
     Fq1Mat m[kFq1Max];
     uint32_t start[kFq1Max];     // first tile index (x) of each product, 0xffffffff past the last
@@ -1666,7 +1666,7 @@ struct Fq1Params {
 };
 
 template <int TYPE, int MAXM>
-__global__ __launch_bounds__(512) void k_gemv_fq1(Fq1Params p) {
+__global__ __launch_bounds__(1024) void k_gemv_fq1(Fq1Params p) {
     using T = GV<TYPE>;
     constexpr int VDT = (TYPE == QMM_TYPE_Q4_0 || TYPE == QMM_TYPE_Q8_0 || TYPE == QMM_TYPE_IQ4_NL) ? QMM_TYPE_Q8_0
                                                                                                      : QMM_TYPE_Q8_K;
@@ -1777,7 +1777,7 @@ bool gemv_fused_slot_plan(int type, const WView & w, int64_t nslots, int64_t T, 
 int64_t gemv_fq1_tree_words(const Fq1Mat & m) { return m.KS > 1 ? (m.M + kTileRows - 1) / kTileRows * 2 * m.KS * 64 : 0; }
 
 hipError_t launch_gemv_fq1(int type, const Fq1Mat * m, int n, int W, const void * sink, hipStream_t s, const KTime * kt) {
-    if (n < 1 || n > kFq1Max || W < 1 || W > 8 || !sink) return hipErrorInvalidValue;
+    if (n < 1 || n > kFq1Max || W < 1 || W > kFqMaxWaves || !sink) return hipErrorInvalidValue;
     Fq1Params p{};
     p.sink = (const uint8_t *)sink;
     p.W = W;

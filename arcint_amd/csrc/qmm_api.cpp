@@ -1122,14 +1122,15 @@ int qmm_describe_mul_mat(const qmm_tensor * src0, const qmm_tensor * src1, const
     return QMM_OK;
 }
 
-// A split-form product of one column and batch, one group a wave, takes k_gemv_fq1 (the same sums, and
+// A product of one column and batch on a plan of one group a wave may run on k_gemv_fq1: in
+// a run of a graph's nodes, and on the split plan by itself too (the same sums, and
 // nothing in the kernel beside them: Q4_0 4096 x 4096 4.95 -> 4.28 us, Q6_K 5120 x 17408 15.3-15.8 ->
 // 14.8, IQ4_XS 4096 x 14336 10.3 -> 9.45, Q4_K 17408 x 5120 10.8-11.0 -> 10.6), but for Q6_K images past
 // the 256 MB Infinity Cache: at 75 registers against 100 six of its waves share a SIMD, not four, and
 // their two-stage requests queue up (151936 x 5120, 638 MB: 97.5 us against 95.9; 40000 x 5120, 168 MB,
 // the same; Q4_K of 350 MB 58.0 against 58.6).  QMM_GEMV_FQ1=0: never.
 static bool fq1_for(int type, const WView & w, const FusedPlan & fp) {
-    return fp.nc == 1 && fp.ntasks == 1 && fp.spw == 1 && fp.KS > 1 && fp.W <= 8 && env_or("QMM_GEMV_FQ1", 1) != 0 &&
+    return fp.nc == 1 && fp.ntasks == 1 && fp.spw == 1 && env_or("QMM_GEMV_FQ1", 1) != 0 &&
            (type != QMM_TYPE_Q6_K || w.ntiles * w.G * (int64_t)w.tg < ((int64_t)256 << 20));
 }
 static Fq1Mat fq1_mat(const qmm_tensor * src1, const WView & w, float * d, int W, uint32_t * tree) {
@@ -2214,7 +2215,10 @@ int qmm_internal_gemv_extent(int32_t type, const int64_t ne0[4], int64_t N, int6
 }
 
 // The run of one-column MUL_MAT nodes from nodes[0] that one k_gemv_fq1 launch takes: one weight type,
-// each on the one-column split or one-slice plan, none reading or writing what another writes.
+// plans of one group a wave in work-groups of as many waves (split, or K whole in one), none reading or
+// writing what another writes.  Each keeps its own plan, and so its order of sums: its bits do not
+// depend on its neighbours in the graph.  One-slice plans in a run, against node by node: 2 x 14336 x
+// 4096 IQ4_XS 16.9 -> 13.1 us, Q4_K 14.1 -> 10.5; 3 x 512 x 2048 Q4_K 14.3 -> 8.0, Q8_0 14.4 -> 8.1.
 // Returns how many (0 or 1: none, run node by node).  A run's slots stay within kTreeMinWords, which
 // every context with slots has, so no run makes the slots grow (and captured graphs void) or, under
 // a capture, need more than a context that ran any split product has.  Kernel timing stamps every
@@ -2229,14 +2233,12 @@ static int fq1_run(qmm_ctx * ctx, const qmm_node * nodes, int n_nodes, Fq1Mat * 
         if (a.op != QMM_OP_MUL_MAT || !mul_mat_ok(a.src0, a.src1, a.dst, true, &w, nullptr, 0)) break;
         const int type = a.src0->type;
         if (a.src1->ne[1] != 1 || a.src1->ne[2] * a.src1->ne[3] != 1 || (n && type != nodes[0].src0->type)) break;
+        // the node's own plan, in the run's waves: its sums are then those it has alone
         FusedPlan fp;
-        if (use_gemm_for(type, w, 1, 1) || !fused_dense_plan(type, w, 1, 1, &fp, true) || fp.nc != 1) break;
-        const int wv = type == QMM_TYPE_Q8_0 ? 8 : 4;
-        FusedPlan split;
-        if (!gemv_fused_split_plan(type, w, 1, 1, wv, 1, &split) || !fq1_for(type, w, split)) break;
-        // (a plan forced by the tuning switches stays as forced)
-        if (fp.KS > 1 && (fp.W != wv || fp.spw != 1)) break;
-        m[n] = fq1_mat(a.src1, w, (float *)((uint8_t *)a.dst->buffer->ptr + a.dst->offs), wv, nullptr);
+        if (use_gemm_for(type, w, 1, 1) || !fused_dense_plan(type, w, 1, 1, &fp, true) || !fq1_for(type, w, fp) ||
+            (n && fp.W != *W))
+            break;
+        m[n] = fq1_mat(a.src1, w, (float *)((uint8_t *)a.dst->buffer->ptr + a.dst->offs), fp.W, nullptr);
         const size_t need = (size_t)gemv_fq1_tree_words(m[n]);
         if (words + need > kTreeMinWords) break;
         bool apart = !ranges_overlap(a.dst, a.src1);
@@ -2254,7 +2256,7 @@ static int fq1_run(qmm_ctx * ctx, const qmm_node * nodes, int n_nodes, Fq1Mat * 
         if (!apart) break;
         m[n].tree = reinterpret_cast<uint32_t *>(words);            // (its offset, until the slots are there)
         words += need;
-        *W = wv;
+        *W = fp.W;
     }
     if (n < 2) return 0;
     if (words) {

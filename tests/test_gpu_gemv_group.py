@@ -99,3 +99,25 @@ def test_group_captured(be, sc, orc):
             assert rel_err(v.reshape(1, M), orc.mul_mat(q, raw, M, K, x)) <= TOL
             assert np.array_equal(v.view(np.uint32), be.get_f32(n[4]).view(np.uint32))
     g.free()
+
+
+# K of 3 to 8 groups whole in one work-group (every order of sums that differs from the split plan's), and
+# 14336 x 4096's one-slice plan of 16 waves (Q6_K's stays split): a run keeps each node's own plan
+@pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("shapes", [[(70, 768), (130, 768)], [(512, 1536), (64, 1536), (100, 1536)],
+                                    [(512, 2048), (256, 2048), (300, 2304), (100, 2048)], [(14336, 4096)] * 2])
+def test_group_keeps_each_plans_sums(be, sc, orc, monkeypatch, qtype, shapes):
+    say("group one-slice", qtype, shapes)
+    nodes, refs = build(be, sc, qtype, shapes, 681)
+    out = []
+    for env in ("1", "0"):
+        monkeypatch.setenv("QMM_GEMV_GROUP", env)
+        for n in nodes:
+            be.set_tensor(n[4], np.zeros(n[4].ne[0], np.float32))
+        be.graph_compute(nodes)
+        be.synchronize()
+        out.append([be.get_f32(n[4]).copy() for n in nodes])
+    for i, (raw, M, K, x) in enumerate(refs):
+        assert np.array_equal(out[0][i].view(np.uint32), out[1][i].view(np.uint32)), (M, K)
+        if M < 1000:
+            assert rel_err(out[0][i].reshape(1, M), orc.mul_mat(qtype, raw, M, K, x)) <= TOL, (M, K)
