@@ -942,18 +942,30 @@ static bool use_gemm_for(int type, const WView & w, int64_t N, int64_t nbatch, b
 }
 
 // A gate/up pair on the GEMM (one launch of both products): past one pass of the GEMV, when its
-// estimated time is below that of the GEMV's passes (32 columns each on the MFMA GEMV, 8 on v_dot4):
-// both images streamed once a pass at 2.7 MB a us, 1.3 us a pass beside that, and the GLU launch's 3
-// us more.  Measured (op us, GEMV / GEMM): Q6_K 11008 x 4096 at N = 77 84 / 43, at 203 162 / 73; Q8_0
-// 2048 x 1024 at 40 11.9 / 15.4, at 128 17.4 / 16.0; Q4_K 17408 x 5120 at 40 (two products) 83 / 46.
+// estimated op time is below that of the GEMV (pre-pass, one launch that streams both images once a
+// pass of 32 columns, 8 on v_dot4, and the GLU kernel).  Both are linear fits by type over 1400 pairs (192-
+// 18432 rows, K 512-7168, 16-700 columns) timed on both routes; the GEMM's in its shape's own estimate, the
+// GEMV's in the columns and in the bytes of its passes.  The choice is the faster or within 3 % on 95 % of
+// them.  Measured (op us, GEMV / GEMM): Q8_0 2048 x 1024 at 48 columns 13.2 / 16.4, 4096 x 4096 at 48
+// 24.4 / 33.3, 512 x 2048 at 200 16.4 / 23.2, 2048 x 2048 at 200 27.0 / 23.1; IQ4_XS 1024 x 1024 at 96 13.9 / 16.5; Q4_K 512 x
+// 2048 at 160 15.8 / 19.6, 17408 x 5120 at 40 83 / 46; Q6_K 11008 x 4096 at 77 84 / 43.
 static bool use_gemm_pair(int type, const WView & w, int64_t N, int64_t nbatch, G3Shape * sh) {
     if (N < gemm_min_cols(type)) return false;
     double us = 0;
     if (!gemm3_shape(type, w, N, nbatch, sh, true, &us)) return false;
     if (getenv("QMM_GEMM_MIN_COLS") || nbatch > 1) return nbatch == 1 || use_gemm_for(type, w, N, nbatch);
-    const int64_t per = gemv_mma_supported(type) ? kMmaMaxCols : 8;
-    const double bytes = 2.0 * (double)(w.ntiles * w.G) * (double)w.tg;
-    return us + 2.0 < 3.0 + (double)((N + per - 1) / per) * (1.3 + bytes / 2.7e6);
+    struct Fit { double gemm, step, gemv, col, mb, mb_col; };     // us; us a column, an MB, an MB and column of a pass
+    const Fit f = type == QMM_TYPE_Q4_0   ? Fit{ 10.0, 0.87, 12.6, 0.0113, 0.286, 0.0034 }
+                : type == QMM_TYPE_Q8_0   ? Fit{ 11.4, 1.00, 12.1, 0.0106, 0.180, 0.0012 }
+                : type == QMM_TYPE_Q4_K   ? Fit{ 11.7, 0.88, 12.9, 0.0109, 0.270, 0.0024 }
+                : type == QMM_TYPE_Q5_K   ? Fit{ 11.3, 0.93, 17.6, 0.0196, 0.0, 0.0321 }
+                : type == QMM_TYPE_Q6_K   ? Fit{ 11.5, 0.91, 13.2, 0.0116, 0.236, 0.0024 }
+                : type == QMM_TYPE_IQ4_XS ? Fit{ 11.7, 1.07, 12.6, 0.0124, 0.336, 0.0019 }
+                                          : Fit{ 10.7, 0.97, 12.8, 0.0106, 0.326, 0.0033 };
+    const int64_t per = gemv_mma_supported(type) ? kMmaMaxCols : 8, passes = (N + per - 1) / per;
+    const double mb = 2e-6 * (double)(w.ntiles * w.G) * (double)w.tg * (double)passes, cols = (double)N / (double)passes;
+    const double few = std::min(1.0, (double)w.ntiles / 8);       // (512 rows and up pay in full for a column)
+    return f.gemm + f.step * us < 0.98 * (f.gemv + f.col * (double)N * few + mb * (f.mb + f.mb_col * cols));
 }
 
 // columns per GEMV task: up to 32 on the MFMA kernel (the rows of its A operand), 8 on v_dot4,

@@ -69,3 +69,27 @@ def test_pair_strides_and_batches(be, sc, orc, monkeypatch, qtype):
     a, b = out[0][1], out[1][1]
     assert np.all(a[:, N:, :] == 7.0) and np.all(a[:, :, M:] == 7.0)     # nothing written past the view
     assert rel_err(a[:, :N, :M].reshape(-1, M), b[:, :N, :M].reshape(-1, M)) <= TOL
+
+
+# GEMV or GEMM by the smaller estimate: pairs that measured 12-45 % apart (op us, GEMV / GEMM)
+@pytest.mark.parametrize("qtype,M,K,N,path", [
+    (qmm.Q8_0, 2048, 1024, 40, "glu-fused-gemv-mfma"),            # 13.0 / 16.4
+    (qmm.Q8_0, 4096, 4096, 48, "glu-fused-gemv-mfma"),            # 24.4 / 33.3
+    (qmm.Q8_0, 512, 2048, 200, "glu-fused-gemv-mfma"),            # 16.4 / 23.2
+    (qmm.Q8_0, 2048, 2048, 256, "glu-gemm-stream"),               # 29.6 / 23.3
+    (qmm.Q4_0, 512, 2048, 200, "glu-fused-gemv-mfma"),            # 16.8 / 19.8
+    (qmm.Q4_0, 4096, 2048, 128, "glu-gemm-stream"),               # 29.9 / 19.9
+    (qmm.Q4_K, 512, 2048, 160, "glu-fused-gemv-mfma"),            # 15.8 / 19.6
+    (qmm.Q4_K, 4096, 2048, 128, "glu-gemm-stream"),               # 29.0 / 19.9
+    (qmm.Q5_K, 2048, 1024, 48, "glu-gemm-stream"),                # 23.7 / 15.9
+    (qmm.Q6_K, 512, 2048, 160, "glu-fused-gemv-mfma"),            # 16.6 / 19.7
+    (qmm.Q6_K, 2048, 2048, 200, "glu-gemm-stream"),               # 31.5 / 20.1
+    (qmm.IQ4_XS, 1024, 1024, 96, "glu-fused-gemv-mfma"),          # 13.9 / 16.5
+    (qmm.IQ4_XS, 4096, 2048, 128, "glu-gemm-stream"),             # 29.4 / 21.6
+    (qmm.IQ4_NL, 512, 2048, 160, "glu-fused-gemv-mfma"),          # 16.6 / 21.6
+    (qmm.IQ4_NL, 2048, 2048, 200, "glu-gemm-stream")])            # 28.2 / 22.3
+def test_pair_rule(be, sc, orc, qtype, M, K, N, path):
+    say("pair rule", qtype, M, K, N)
+    got, ref = glu_case(be, sc, orc, qtype, qtype, M, K, N, qmm.GLU_SWIGLU, seed=541)
+    assert be.last_path() == path
+    assert rel_err(got, ref) <= TOL
