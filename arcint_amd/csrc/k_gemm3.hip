@@ -1762,8 +1762,10 @@ bool kq_shape(int type, const WView & w, int64_t N, int64_t nbatch, G3Shape * sh
 //    the 32-weight ones).
 //  * 12-wave blocks run one a CU in whole rounds, 4-wave ones up to three a CU.
 //  * One-slice launches of a block per CU or more may run the blocks past a whole number per CU as
-//    2-4 pieces along K: the pieces' sums pass through memory as 64-bit exchanges, 1.6 us a MB (11008 x
-//    4096 Q4_0, N = 203: 704 pieces, 98 us, against 68 us with 12-wave whole blocks).
+//    2-4 pieces along K: the pieces' sums pass through memory as 64-bit exchanges, whose two round trips
+//    after the last step cost 10 us whatever their number, and 0.9 us a MB.  Measured (op us, pieces /
+//    whole): IQ4_XS 10992 x 1280 at 140 columns (512 + 4 blocks) 50.9 / 35.5, Q4_0 16764 x 1536 at 77 44.0 /
+//    33.0, 11008 x 4096 at 203 (704 pieces) 98 / 68; of 120 shapes with a tail 34 gain from them.
 // Measured at (U, KS) = (12, 1) / (6, 2) / (4, 3) / (4, 1) / (2, 2), op us, the estimate's choice first
 // or within 4 % of it: Q4_K 17408 x 5120, N = 77 186 / 90 / 100 / 75 / 83, N = 203 152 / 139 / 166 /
 // 130 / 144, N = 512 247 / 274 / 305 / 234 / 276; Q4_0 11008 x 4096, N = 40 66 / 39 / 31 / 59 / 33, N =
@@ -1773,6 +1775,7 @@ bool kq_pair_shape(const WView & w, int64_t N, int64_t nbatch, G3Shape * sh, boo
     static const Cand cands[] = { { 12, 1, 1 }, { 6, 2, 1 }, { 4, 3, 1 }, { 4, 1, 3 }, { 2, 2, 3 } };
     const int64_t ncp = ((N + 31) / 32 + 1) / 2, nrh = 2 * w.ntiles, G = w.G, cus = 256;
     const int forced = env_int3("QMM_GEMM3_PAIR", -1);         // index into cands (tuning)
+    const int tail = env_int3("QMM_GEMM3_TAIL", 1);            // 0: whole blocks, 2..4: that many pieces (tuning)
     const double c = blk ? 1.3 : 1.1;
     auto t = [](double waves) { return waves <= 1 ? 2.0 : waves <= 2 ? 1.6 + 0.4 * waves : 0.68 + 0.86 * waves; };
     double best = -1;
@@ -1790,13 +1793,13 @@ bool kq_pair_shape(const WView & w, int64_t N, int64_t nbatch, G3Shape * sh, boo
         const double two = cd.U == 2 ? (full + (rest > 0) > 2 ? 1.25 : 1.1) : 1.0;
         double cost = steps((double)(full + (rest > 0))) * c * two;
         int64_t ts = 1;
-        if (KS == 1 && nbatch == 1 && full > 0) {
+        if (KS == 1 && nbatch == 1 && full > 0 && tail != 0) {
             for (int64_t k = 2; k <= 4 && rest > 0; ++k) {
                 const int64_t pk = (G + k - 1) / k;
-                if (pk < 2 || (k - 1) * pk >= G) continue;
+                if (pk < 2 || (k - 1) * pk >= G || (tail > 1 && k != tail)) continue;
                 const double load = (double)full + (double)((rest * k + cus - 1) / cus) / (double)k;
-                const double v = steps(load) * c + (double)(rest * k) * (cd.U / 2) * 0.026;
-                if (v < cost) {
+                const double v = steps(load) * c + 10.0 + (double)(rest * k) * (cd.U / 2) * 0.015;
+                if (v < cost || tail > 1) {
                     cost = v;
                     ts = k;
                 }

@@ -36,6 +36,7 @@ def test_pair_shapes(be, sc, orc, monkeypatch, qtype, shape):
                                         (qmm.Q5_K, 1536, qmm.GLU_GEGLU_ERF)])
 def test_pair_tail_pieces(be, sc, orc, monkeypatch, qtype, K, op):
     monkeypatch.setenv("QMM_GEMM3_PAIR", "3")
+    monkeypatch.setenv("QMM_GEMM3_TAIL", "3" if K == 1536 else "2")
     monkeypatch.setenv("QMM_GEMM_MIN_COLS", "16")
     say("pair-tail", qtype, K, op)
     got, ref = glu_case(be, sc, orc, qtype, qtype, 1850, K, 561, op, seed=521)
@@ -93,3 +94,33 @@ def test_pair_rule(be, sc, orc, qtype, M, K, N, path):
     got, ref = glu_case(be, sc, orc, qtype, qtype, M, K, N, qmm.GLU_SWIGLU, seed=541)
     assert be.last_path() == path
     assert rel_err(got, ref) <= TOL
+
+
+def test_pair_captured_without_slots(orc, monkeypatch):
+    """a pair whose launch has tail pieces, captured by a context that has no exchange slots: the blocks run
+    whole, in every replay, with eager work between them"""
+    say("pair captured cold")
+    monkeypatch.setenv("QMM_GEMM3_PAIR", "3")
+    monkeypatch.setenv("QMM_GEMM3_TAIL", "0")
+    monkeypatch.setenv("QMM_GEMM_MIN_COLS", "16")
+    q, M, K, N = qmm.Q4_K, 1850, 1024, 561                        # 256 + 5 blocks
+    with qmm.Backend(0) as be:
+        s = Scope(be)
+        w = [s.weights(q, synth.weights(q, M, K, seed=551 + i), (K, M)) for i in range(2)]
+        xs = [synth.activations(N, K, seed=555 + i) for i in range(3)]
+        x, y, z = s.f32(xs[0]), s.empty_f32((M, N)), s.empty_f32((M, N))
+        be.mul_mat_glu(w[0], w[1], x, y, qmm.GLU_SWIGLU)          # (whole: scratch for the activations, no slots)
+        be.synchronize()
+        monkeypatch.setenv("QMM_GEMM3_TAIL", "2")
+        be.capture_begin()
+        be.mul_mat_glu(w[0], w[1], x, y, qmm.GLU_SWIGLU)
+        g = be.capture_end()
+        monkeypatch.setenv("QMM_GEMM3_TAIL", "0")
+        for v in xs:
+            be.set_tensor(x, v.view(np.uint8).ravel())
+            be.graph_launch(g)
+            be.mul_mat_glu(w[0], w[1], x, z, qmm.GLU_SWIGLU)      # eager, whole blocks: the same sums
+            be.synchronize()
+            assert np.array_equal(be.get_f32(y).view(np.uint32), be.get_f32(z).view(np.uint32))
+        g.free()
+        s.close()
