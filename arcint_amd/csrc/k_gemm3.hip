@@ -1557,21 +1557,37 @@ __global__ __launch_bounds__(64 * kWideU, 2) void k_gemm3_wide(KQParams p) {
 
     if (!row_ok) return;
     constexpr float scale = TYPE == QMM_TYPE_Q4_0 ? 0.0625f : 1.0f;   // (Q4_0 codes carried 16 (q - 8))
-#pragma unroll
-    for (int i = PAIR ? 1 : 0; i < 2; ++i) {
-        const int64_t m = mtile * kTileRows + 32 * (PAIR ? t : i) + j32;
-        if (m >= p.w.M) continue;
+    if constexpr (PAIR) {
+        const int64_t m = mtile * kTileRows + 32 * t + j32;
+        if (m >= p.w.M) return;
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
             float gv[16], val[16];
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                val[r] = out[i][c][r] * scale;
                 gv[r] = out[0][c][r] * scale;
+                val[r] = out[1][c][r] * scale;
             }
-            if constexpr (PAIR) glu_switch(p.glu, gv, val);
+            glu_switch(p.glu, gv, val);
             kq_store(p, nb, c, i2, i3, m, h, 0xffffu, val);
         }
+    } else {
+        // both row halves of a column one after the other: 64 rows, 256 bytes.  Where rows of dst do not begin on a
+        // cache line, two half-lines that meet in L2 are one write to memory; stored 32 columns apart they
+        // were two (Q8_0 12222 x 544 at 1329 columns 69 -> 51 us, 12224 x 544 43.3 -> 44.4; IQ4_NL 57678 x 512 at
+        // 691 147 -> 91; Q4_0 8191 x 4096 at 1024 97.9 -> 94.1)
+        const int64_t m = mtile * kTileRows + j32;
+        const bool lo = m < p.w.M, hi = m + 32 < p.w.M;
+        float * dst = p.dst + (int64_t)i2 * p.bt.d_nb2 + (int64_t)i3 * p.bt.d_nb3 + m;
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int64_t n = (2 * (int64_t)nb + c) * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+                if (n >= p.N) continue;
+                if (lo) __builtin_nontemporal_store(out[0][c][r] * scale, dst + n * p.bt.d_nb1);
+                if (hi) __builtin_nontemporal_store(out[1][c][r] * scale, dst + n * p.bt.d_nb1 + 32);
+            }
     }
 }
 
@@ -1854,15 +1870,21 @@ bool kq_pair_shape(const WView & w, int64_t N, int64_t nbatch, G3Shape * sh, boo
     if (us) *us = best;
     return best >= 0 && sh->mbn * ncp < 0x7fffffff && sh->lds <= 160 * 1024 && sh->threads <= 64 * kKQMaxWaves;
 }
-// Launch shape of the 64 x 64 waves (k_gemm3_wide), and whether it is taken: when its estimated time is
-// below that of 32-row waves, us (their own estimate for a gate/up pair, else by their count).  In us a
-// step of 256 weights: two work-groups a CU take w a step; 12 waves of 32 rows a CU take n.  Rounds
-// of 512 work-groups: up to 256 left over run one a CU, in about half a round (a lone work-group has
-// the CU to itself), more of them nearly a whole one.  Measured (8192 x 4096, wide / narrow us): Q4_0
-// 1024 columns (1 round) 87 / 101, 1088 (1.06) 131 / 106, 1408 (1.38) 133 / 128, 1536 (1.5) 134 / 139,
-// 1664 (1.63) 157 / 153, 2048 (2) 167 / 186; Q8_0 1024 87 / 114, 1280 (1.25) 131 / 131, 1536 134 / 155;
-// IQ4_NL 768 (0.75) 90 / 85, 1024 100 / 115; FFN blocks by pairs: Q4_0 256 columns (0.5) 101 / 96, 448 137 /
-// 157, 576 (1.13) 200 / 189, 768 (1.5) 228 / 235, Q8_0 256 100 / 111, 512 150 / 187.
+// Launch shape of the 64 x 64 waves (k_gemm3_wide), and whether it is taken: when its estimated op time
+// is below that of 32-row waves (for a gate/up pair their own estimate of the steps, us).  In us:
+//  * a step of 256 weights takes two work-groups a CU w, and 12 waves of 32 rows a CU n.  Rounds of 512
+//    work-groups: up to 256 left over run one a CU, in about half a round (a lone work-group has the CU
+//    to itself), more of them nearly a whole one;
+//  * one product: beside its steps the wide launch takes 9.2 us and 0.15 a MB of dst (its waves all store
+//    at once, and two a SIMD hide less of it), the narrow one 14.5 and 0.6 a round.  2 us and 1 % more for the
+//    estimates' error.  Where K is short the stores decide: Q4_0 13756 x 768 at 836 columns 44 / 38 (wide /
+//    narrow), 31219 x 544 at 360 42 / 36, 39216 x 512 at 1961 150 / 144; IQ4_NL 16884 x 896 at 669 53 / 50; Q8_0 12838 x
+//    512 at 790 34 / 31.  Over 700 shapes of 512-8192 weights a row and 33-2048 columns the choice loses 3 %
+//    to the narrow waves at most (the steps alone: 18 %, and more than 3 % on 21 shapes).
+// Measured (8192 x 4096, wide / narrow us): Q4_0 1024 columns (1 round) 87 / 101, 1088 (1.06) 131 / 106, 1408
+// (1.38) 133 / 128, 1536 (1.5) 134 / 139, 1664 (1.63) 157 / 153, 2048 (2) 167 / 186; Q8_0 1024 87 / 114, 1280
+// (1.25) 131 / 131, 1536 134 / 155; IQ4_NL 768 (0.75) 90 / 85, 1024 100 / 115; FFN blocks by pairs: Q4_0 256
+// columns (0.5) 101 / 96, 448 137 / 157, 576 (1.13) 200 / 189, 768 (1.5) 228 / 235, Q8_0 256 100 / 111, 512 150 / 187.
 bool kq_wide_shape(int type, const WView & w, int64_t N, int64_t nbatch, G3Shape * sh, bool pair, double us) {
     const int64_t ncp = ((N + 31) / 32 + 1) / 2, units = pair ? 2 * w.ntiles : w.ntiles;
     const int64_t mbn = (units + kWideU - 1) / kWideU, nwg = mbn * ncp;
@@ -1870,13 +1892,17 @@ bool kq_wide_shape(int type, const WView & w, int64_t N, int64_t nbatch, G3Shape
     if (env == 0 || (env < 0 && env_int3(pair ? "QMM_GEMM3_PAIR" : "QMM_GEMM3_KQ", -1) >= 0)) return false;
     if (env < 0) {
         const bool q4 = type == QMM_TYPE_Q4_0, q8 = type == QMM_TYPE_Q8_0;
-        const double wstep = q4 ? 5.2 : q8 ? 5.1 : 5.75, nstep = q4 ? 4.36 : q8 ? 5.0 : 4.95;
+        const double G = (double)w.G;
         const int64_t whole = nwg * nbatch / 512, rest = nwg * nbatch % 512;
-        const double rounds = (double)whole + (rest == 0 ? 0 : whole == 0 ? (rest <= 256 ? 0.66 : 1.0) : rest <= 256 ? 0.55 : 0.9);
-        // (a pair's own estimate is at Q4_0's 4.25 a step)
-        const double narrow = pair ? us * (q4 ? 1.0 : nstep / 4.25)
-                                   : (double)(2 * w.ntiles * ncp * nbatch) / 3072 * nstep * (double)w.G;
-        if (rounds * wstep * (double)w.G > 0.975 * narrow) return false;
+        const double rounds = (double)whole + (rest == 0 ? 0 : whole == 0 ? (rest <= 256 ? 0.66 : 1.0) : rest <= 256 ? 0.6 : 0.9);
+        if (pair) {
+            const double wstep = q4 ? 5.2 : q8 ? 5.1 : 5.75, nstep = q4 ? 1.0 : q8 ? 5.0 / 4.25 : 4.95 / 4.25;
+            if (rounds * wstep * G > 0.975 * us * nstep) return false;   // (us is at Q4_0's step)
+        } else {
+            const double wstep = q4 ? 4.65 : q8 ? 4.55 : 5.48, nstep = q4 ? 3.96 : q8 ? 4.5 : 4.57;
+            const double nrounds = (double)(2 * w.ntiles * ncp * nbatch) / 3072, mb = 4e-6 * (double)(w.M * N * nbatch);
+            if (11.2 + rounds * wstep * G + 0.15 * mb > 0.99 * (14.5 + nrounds * (0.6 + nstep * G))) return false;
+        }
     }
     *sh = G3Shape{};
     sh->C = 2;

@@ -71,3 +71,20 @@ def test_wide_rule(qtype, N, wide):
         assert (info["threads"], info["workgroups"], info["lds_bytes"]) == (256, 32 * pairs, 37 * 1024)
     else:
         assert (info["threads"], info["workgroups"]) != (256, 32 * pairs)
+
+
+# short K, where the stores decide (op us, 64-row / 32-row waves)
+@pytest.mark.parametrize("qtype,M,K,N,wide", [(qmm.Q4_0, 13756, 768, 836, False),        # 44 / 38
+                                              (qmm.Q4_0, 39216, 512, 1961, False),       # 150 / 144
+                                              (qmm.Q4_0, 31219, 544, 360, False),        # 42 / 36
+                                              (qmm.IQ4_NL, 16884, 896, 669, False),      # 53 / 50
+                                              (qmm.Q8_0, 12838, 512, 790, False),        # 34 / 31
+                                              (qmm.Q8_0, 12222, 544, 1329, True),        # 51 / 55
+                                              (qmm.Q8_0, 16384, 4096, 512, True),        # 97 / 121
+                                              (qmm.Q4_0, 4096, 11008, 2048, True)])      # 247 / 275
+def test_wide_rule_short_k(qtype, M, K, N, wide):
+    fake = qmm.Buffer(ptr=0x1000, size=1 << 44)
+    info = qmm.describe_mul_mat(qmm.Tensor(fake, qtype, (K, M)), qmm.Tensor(fake, qmm.F32, (K, N)),
+                                qmm.Tensor(fake, qmm.F32, (M, N)))
+    groups = -(-M // 256) * -(-N // 64)
+    assert ((info["threads"], info["lds_bytes"]) == (256, 37 * 1024) and info["workgroups"] == -(-groups // 8) * 8) == wide
