@@ -924,12 +924,12 @@ static double gemv_passes_us(int type, const WView & w, int64_t N) {
 // 40-64 44.7-50.8 / 31, 12288 x 5120 at 48 30.0 / 30.0, 5120 x 6144 at 48-64 22-24 / 32-33; the Q6_K
 // 151936-row head at 64 446 / 272; Q5_K 17408 x 5120 at 16-48 62-135 / 34-36; config 3's shared expert
 // (Q4_K 512 x 2048, N = 256) 30.4 / 42.8.  QMM_GEMM_MIN_COLS, when set, decides alone.
-static bool use_gemm_for(int type, const WView & w, int64_t N, int64_t nbatch, bool whole = false) {
+static bool use_gemm_for(int type, const WView & w, int64_t N, int64_t nbatch) {
     if (N < gemm_min_cols(type)) return false;
     if (getenv("QMM_GEMM_MIN_COLS")) return true;
     G3Shape sh;
     double us = -1;
-    if (!gemm3_shape(type, w, N, nbatch, &sh, false, &us, whole)) return true;      // (the shared-tile GEMM)
+    if (!gemm3_shape(type, w, N, nbatch, &sh, false, &us)) return true;             // (the shared-tile GEMM)
     if (us >= 0) gemm3_shape(type, w, N, nbatch, &sh, false, nullptr, true);        // (the rounds' launch)
     const int64_t waves = sh.mbn * sh.nbn * nbatch * sh.U * sh.KS;
     const int64_t per = gemv_mma_supported(type) ? kMmaMaxCols : 8;
@@ -1224,8 +1224,10 @@ static bool try_fused_id(qmm_ctx * ctx, const qmm_tensor * src0, const qmm_tenso
 static int mul_mat_launch(qmm_ctx * ctx, const qmm_tensor * src0, const qmm_tensor * src1, const qmm_tensor * dst,
                           const WView & w, const FixedAct * fixed) {
     const int64_t N = src1->ne[1];
-    const bool whole = fixed || gemm_whole(ctx, src0->type, w, N, src1->ne[2] * src1->ne[3]);
-    const bool use_gemm = use_gemm_for(src0->type, w, N, src1->ne[2] * src1->ne[3], whole);
+    // (the path is qmm_describe_mul_mat's whether or not the GEMM's tail pieces have slots: a capture then
+    // finds the scratch of the same op run before it)
+    const bool use_gemm = use_gemm_for(src0->type, w, N, src1->ne[2] * src1->ne[3]);
+    const bool whole = use_gemm && (fixed || gemm_whole(ctx, src0->type, w, N, src1->ne[2] * src1->ne[3]));
     ActBuf a{};
     int rc;
     float * d = (float *)((uint8_t *)dst->buffer->ptr + dst->offs);
@@ -1242,8 +1244,8 @@ static int mul_mat_launch(qmm_ctx * ctx, const qmm_tensor * src0, const qmm_tens
     KTime kt;
     const KTime * ktp = nullptr;
     G3Shape g3;
-    // weights streamed per wave, dst written once (the shape check is qmm_describe_mul_mat's, so
-    // a shape the streaming kernel declines runs on the shared-tile GEMM below, as described)
+    // weights streamed per wave, dst written once (a shape the streaming kernel declines runs on the
+    // shared-tile GEMM below, as qmm_describe_mul_mat says)
     if (use_gemm && gemm3_shape(src0->type, w, N, dn.ne12 * dn.ne13, &g3, false, nullptr, whole)) {
         const int64_t nbatch = dn.ne12 * dn.ne13;
         TiledAct ta;

@@ -370,7 +370,9 @@ int64_t qmm_downgrades(qmm_ctx * ctx, char * buf, size_t buf_len);
 const char * qmm_last_path(qmm_ctx * ctx);
 
 /* The launch a qmm_mul_mat with these tensors would make (host only, no
- * device, no buffers needed: only types and shapes are read). */
+ * device, no buffers needed: only types and shapes are read).  A "gemm-stream" launch that has no
+ * exchange slots (qmm_mul_mat_noalloc, and a capture that would have to grow them) takes the same
+ * path with whole blocks, in a shape chosen for them. */
 typedef struct qmm_launch_info {
     char    path[32];          /* as qmm_last_path: "gemv", "gemv-mfma", "gemv-fq", "gemm-stream" or
                                   "gemm-mfma" */

@@ -54,3 +54,57 @@ def test_longk_product(be, sc, monkeypatch, qtype, M, K, N):
         got = be.get_f32(full).reshape(N + 1, M + 3)
         assert np.all(got[N:] == 7.0) and np.all(got[:, M:] == 7.0)
         assert rel_err(got[:N, :M], oracle.mul_mat(qtype, raw, M, K, x)) <= TOL
+
+
+# without exchange slots the path is still the described one: the GEMV where it is chosen by time, the GEMM
+# in whole blocks elsewhere
+@pytest.mark.gpu
+@pytest.mark.parametrize("qtype,M,K,N", [(qmm.Q8_0, 4096, 14336, 40), (qmm.Q8_0, 4096, 14336, 128), (qmm.Q5_K, 722, 8704, 308),
+                                         (qmm.IQ4_XS, 4096, 14336, 77)])
+def test_longk_noalloc(be, sc, qtype, M, K, N):
+    say("longk noalloc", qtype, M, K, N)
+    raw, x = synth.weights(qtype, M, K, seed=711), synth.activations(N, K, seed=712)
+    w, xt, ya, yb = sc.weights(qtype, raw, (K, M)), sc.f32(x), sc.empty_f32((M, N)), sc.empty_f32((M, N))
+    path = describe(qtype, K, M, N)["path"]
+    be.mul_mat_noalloc(w, xt, yb)
+    assert be.last_path() == path
+    be.mul_mat(w, xt, ya)
+    assert be.last_path() == path
+    be.synchronize()
+    got = be.get_f32(yb).reshape(N, M)
+    assert rel_err(got, be.get_f32(ya).reshape(N, M)) <= TOL
+    rows = 64
+    assert rel_err(got[:, :rows], oracle.mul_mat(qtype, raw[:raw.size // M * rows], rows, K, x)) <= TOL
+
+
+# a capture by a context without exchange slots, after the op ran once: the eager call's path on the eager
+# call's scratch, whichever it is; replays with eager work between them
+@pytest.mark.gpu
+@pytest.mark.parametrize("qtype,M,K,N,path", [(qmm.Q8_0, 4096, 14336, 40, "gemv-mfma"), (qmm.Q8_0, 4096, 14336, 128, "gemm-stream")])
+def test_longk_captured_without_slots(monkeypatch, qtype, M, K, N, path):
+    say("longk captured cold", qtype, M, K, N)
+    with qmm.Backend(0) as be:
+        s = Scope(be)
+        raw = synth.weights(qtype, M, K, seed=721)
+        w, xs = s.weights(qtype, raw, (K, M)), [synth.activations(N, K, seed=722 + i) for i in range(3)]
+        x, y, z = s.f32(xs[0]), s.empty_f32((M, N)), s.empty_f32((M, N))
+        monkeypatch.setenv("QMM_GEMM3_TAIL", "0" if path == "gemm-stream" else "1")    # (whole blocks: no slots grown)
+        be.mul_mat(w, x, y)
+        be.synchronize()
+        monkeypatch.setenv("QMM_GEMM3_TAIL", "1")
+        be.capture_begin()
+        be.mul_mat(w, x, y)
+        g = be.capture_end()
+        assert be.last_path() == path
+        for v in xs:
+            be.set_tensor(x, v.view(np.uint8).ravel())
+            be.graph_launch(g)
+            be.mul_mat_noalloc(w, x, z)                               # (whole blocks too)
+            be.synchronize()
+            assert be.last_path() == path
+            if path == "gemm-stream":                                 # (the GEMV's K slices meet in any order)
+                assert np.array_equal(be.get_f32(y).view(np.uint32), be.get_f32(z).view(np.uint32))
+            assert rel_err(be.get_f32(y).reshape(N, M), be.get_f32(z).reshape(N, M)) <= TOL
+            assert rel_err(be.get_f32(y).reshape(N, M)[:, :64], oracle.mul_mat(qtype, raw[:raw.size // M * 64], 64, K, v)) <= TOL
+        g.free()
+        s.close()
