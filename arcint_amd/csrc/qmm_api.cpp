@@ -2291,9 +2291,9 @@ int qmm_graph_compute(qmm_ctx * ctx, const qmm_node * nodes, int n_nodes) {
         Fq1Mat m[kFq1Max];
         int W = 0;
         if (n.op == QMM_OP_MUL_MAT && n.src1 && n.src1->ne[1] == 1 && i + 1 < n_nodes &&
+            hipSetDevice(ctx->device) == hipSuccess &&            // (fq1_run may allocate the slots)
             (done = fq1_run(ctx, nodes + i, n_nodes - i, m, &W)) > 1) {
-            rc = hipSetDevice(ctx->device) == hipSuccess ? fq1_launch(ctx, n.src0->type, m, done, W)
-                                                         : fail(ctx, QMM_ERR_DEVICE, "graph_compute: hipSetDevice");
+            rc = fq1_launch(ctx, n.src0->type, m, done, W);
             ctx->path = "gemv-fq";
         } else {
             done = 1;
