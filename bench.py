@@ -594,9 +594,9 @@ def main():
         # one launch (the fused kernel quantizes its own activations, K over 4-wave work-groups)
         # or the q8_K pre-pass and the GEMV
         fused = path == "gemv-fq"
-        tag = "q4k_gemv_fq" if fused else "q4k_gemv"
-        prof = "profiles/k_gemv_fq_q4k_17408x5120_n1.md" if fused else "profiles/k_gemv_q4k_17408x5120_n1.md"
-        kname = ("k_gemv_fq<12, 1> (Q4_K, 1 column, K split over 4-wave work-groups, activations quantized "
+        tag = "q4k_gemv_fq1" if fused else "q4k_gemv"
+        prof = "profiles/k_gemv_fq1_q4k_17408x5120_n1.md" if fused else "profiles/k_gemv_q4k_17408x5120_n1.md"
+        kname = ("k_gemv_fq1<12, 1> (Q4_K, 1 column, K split over 4-wave work-groups, activations quantized "
                  "in the kernel)" if fused else "k_gemv<12, 1> (Q4_K, 1 column)")
         op_desc = "MUL_MAT in one launch" if fused else "MUL_MAT incl. q8_K pre-pass"
         traffic = profile_traffic(tag)
