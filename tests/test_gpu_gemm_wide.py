@@ -56,6 +56,31 @@ def test_wide_pair(be, sc, orc, monkeypatch, qtype, op):
         assert rel_err(got, ref) <= TOL, (M, K, N)
 
 
+# a pair over batches that share weights, dst columns and batches padded, columns of src1 at a stride: against the
+# 32-row waves (the same sums in the same order), rows and columns past a tile
+@pytest.mark.gpu
+@pytest.mark.parametrize("qtype", BLOCKS)
+def test_wide_pair_strides_and_batches(be, sc, monkeypatch, qtype):
+    K, M, N, B = 544, 97, 75, 4
+    say("wide pair strides", qtype)
+    monkeypatch.setenv("QMM_GEMM_MIN_COLS", "16")
+    w = [sc.weights(qtype, synth.weights(qtype, 2 * M, K, seed=631 + i), (K, M, 2)) for i in range(2)]
+    x = sc.f32(synth.activations(B * 2 * N, K, seed=633).reshape(B, 2 * N, K)).view((K, N, B), (4, 8 * K, 8 * K * N, 8 * K * N * B))
+    out = []
+    for env in ({"QMM_GEMM3_WIDE": "1"}, {"QMM_GEMM3_WIDE": "0", "QMM_GEMM3_PAIR": "0"}):
+        with monkeypatch.context() as mp:
+            for k, v in env.items():
+                mp.setenv(k, v)
+            full = sc.f32(np.full((B, N + 3, M + 5), 7.0, np.float32))
+            nb1 = 4 * (M + 5)
+            be.mul_mat_glu(w[0], w[1], x, full.view((M, N, B), (4, nb1, nb1 * (N + 3), nb1 * (N + 3) * B)), qmm.GLU_SWIGLU)
+            be.synchronize()
+            assert be.last_path() == "glu-gemm-stream"
+            out.append(be.get_f32(full).reshape(B, N + 3, M + 5))
+    assert np.all(out[0][:, N:, :] == 7.0) and np.all(out[0][:, :, M:] == 7.0)     # nothing written past the view
+    assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
+
+
 # the launch rule: 64-row waves from about a round of 512 work-groups on, not where most of a further
 # round would be empty (r rounds of 128 row tiles x 64-column pairs), and not for the other types
 @pytest.mark.parametrize("qtype,N,wide", [(qmm.Q4_0, 64, False), (qmm.Q4_0, 768, False), (qmm.Q4_0, 1024, True),
