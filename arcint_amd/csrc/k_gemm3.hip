@@ -1394,10 +1394,9 @@ __global__ __launch_bounds__(64 * kKQMaxWaves) void k_gemm3_blk(KQParams p) {
 // ---- Q4_0, Q8_0, IQ4_NL, large launches: waves of 64 rows x 64 columns ----------------------
 // k_gemm3_blk's step on two row units a wave: both halves of an image tile, or (PAIR) one half of the
 // gate's tile and the same half of up's, so a pair's two sums meet in the lane's registers.  Bound by
-// the work each block-tile issues, which adds up at the chip's sustained power (per SIMD: an MFMA 18.5
-// ns, a VALU instruction 0.85, an LDS read of 16 bytes a lane 6.3): k_gemm3_blk's 37 VALU and 5 LDS
-// reads a block-tile are 84 ns, and 4 of the 5 reads bring the column scales.  Here one read of the
-// operand and of the scales serves both row units: 2.5 a block-tile.
+// the work each block-tile issues: k_gemm3_blk's 38 VALU instructions and 5 LDS reads an MFMA, 4 of the 5 for
+// the column scales.  Here one read of the operand and of the scales serves both row units, 2.5 an MFMA, and
+// one unit's VALU work overlaps the other's MFMA (0.63 of the matrix cores' busy cycles, 0.41 before).
 //  * 4 waves a work-group (one stage, one K slice), two work-groups a CU: two waves a SIMD with up to
 //    256 registers (64 sums, 32 MFMA results, 32 of weights: PF = 4 blocks ahead instead of 8).
 //  * Measured, op us, against k_gemm3_blk: Q4_0 11008 x 4096 x 2048 250 -> 239, 4096 x 11008 x 2048

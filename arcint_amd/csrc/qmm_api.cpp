@@ -1429,11 +1429,12 @@ static int route_units(qmm_ctx * ctx, const qmm_tensor * ids, int64_t ne11, int6
 }
 
 // MUL_MAT_ID on the grouped GEMM when the experts average this many pairs or more
-// (QMM_MOE_GEMM_MIN overrides; 0 switches it off).  Gate + up + GLU on Q4_K from 64: its GEMV
-// tasks fuse both products and the GLU in one launch on the MFMA GEMV, which the grouped GEMM's
-// route and two launches overtake only past ~60 pairs (16 experts of 512 x 2048, top-10: 37.3
-// against 30.7 us at 40 pairs, 40.2 against 44.1 at 80; IQ4_XS breaks even at 40, Q5_K's v_dot4
-// tasks lose from 25)
+// (QMM_MOE_GEMM_MIN overrides; 0 switches it off).  Gate + up + GLU on Q4_K from 64: the line was drawn
+// when the grouped GEMM took the pair in two launches (16 experts of 512 x 2048, top-10: 37.3 us against
+// the GEMV tasks' 30.7 at 40 pairs).  In the one launch it takes now it is ahead from 24-32 pairs on (24.7
+// against 30.5 there; 128 experts top-8 at 32 pairs 85 / 118; Q6_K 96 / 175, Q5_K 96 / 240, IQ4_XS 95 / 137, and
+// behind at 16 for Q4_K and IQ4_XS, 77.5 / 72.8 and 88 / 84): the line has room below 64, and below 32 for Q6_K and
+// Q5_K
 static int64_t moe_gemm_min_pairs(int type = -1, bool glu = false) {
     const char * e = getenv("QMM_MOE_GEMM_MIN");
     return e ? atoll(e) : glu && type == QMM_TYPE_Q4_K ? 64 : 32;
