@@ -1802,7 +1802,7 @@ bool kq_shape(int type, const WView & w, int64_t N, int64_t nbatch, G3Shape * sh
 //    2-4 pieces along K: the pieces' sums pass through memory as 64-bit exchanges, whose two round trips
 //    after the last step cost 10 us whatever their number, and 0.9 us a MB.  Measured (op us, pieces /
 //    whole): IQ4_XS 10992 x 1280 at 140 columns (512 + 4 blocks) 50.9 / 35.5, Q4_0 16764 x 1536 at 77 44.0 /
-//    33.0, 11008 x 4096 at 203 (704 pieces) 98 / 68; of 120 shapes with a tail 34 gain from them.
+//    33.0, 11008 x 4096 at 203 (704 pieces) 98 / 68; of 120 shapes with a tail 34 still take them.
 // Measured at (U, KS) = (12, 1) / (6, 2) / (4, 3) / (4, 1) / (2, 2), op us, the estimate's choice first
 // or within 4 % of it: Q4_K 17408 x 5120, N = 77 186 / 90 / 100 / 75 / 83, N = 203 152 / 139 / 166 /
 // 130 / 144, N = 512 247 / 274 / 305 / 234 / 276; Q4_0 11008 x 4096, N = 40 66 / 39 / 31 / 59 / 33, N =
